@@ -79,6 +79,7 @@ struct FlashArgs {
     const int* wl;
     float* o_direct;
     float* l_direct;
+    int spread;        // deal the row tiles over the XCDs, longest first (flash_spread)
     // dense unsplit 16-bit pass only (flash_ctx16_ok): instead of o / l, write each row
     // already normalised and rounded to the storage format, (o_scale O) (1 / l) -- what
     // 3d's A staging forms from ctx and row_sum -- at ctx16[row][R]
@@ -98,11 +99,19 @@ struct FlashWork {
 // workgroup i runs on XCD i % 8 in the dispatcher's order, and item t's row tiles are
 // workgroups 8 (row_tiles (t / 8) + rt) + t % 8 -- one XCD per item, the items (longest
 // first) spread over the XCDs in list order, and the unused tail of the grid spread too.
+// With many row tiles per batch (a.spread, flash_spread): spread_tile's order (worklist.h).
 __device__ __forceinline__ FlashWork flash_work(const FlashArgs& a) {
     FlashWork w;
     w.direct = false;
     w.skip = false;
     if (!a.wl) {
+        if (a.spread) {   // n_split == 1
+            spread_tile(blockIdx.x, a.B, a.row_tiles, &w.b, &w.rt);
+            w.k_lo = 0;
+            w.k_len = a.keys_per_split;
+            w.slot = w.b;
+            return w;
+        }
         const int wg = xcd_logical_block(blockIdx.x, gridDim.x);
         const int sp = wg % a.n_split;
         w.rt = (wg / a.n_split) % a.row_tiles;
@@ -112,14 +121,18 @@ __device__ __forceinline__ FlashWork flash_work(const FlashArgs& a) {
         w.slot = (int64_t)sp * a.B + w.b;
         return w;
     }
-    const int x = blockIdx.x % kNumXCDs, q = blockIdx.x / kNumXCDs;
-    const int it = (q / a.row_tiles) * kNumXCDs + x;
-    w.rt = q % a.row_tiles;
-    w.b = 0; w.k_lo = 0; w.k_len = 0; w.slot = 0;
-    if (it >= load_uniform(a.wl)) {
-        w.skip = true;
-        return w;
+    const int n_items = load_uniform(a.wl);
+    int it;
+    w.b = 0; w.k_lo = 0; w.k_len = 0; w.slot = 0; w.rt = 0;
+    if (a.spread) {
+        w.skip = !spread_tile(blockIdx.x, n_items, a.row_tiles, &it, &w.rt);
+    } else {
+        const int x = blockIdx.x % kNumXCDs, q = blockIdx.x / kNumXCDs;
+        it = (q / a.row_tiles) * kNumXCDs + x;
+        w.rt = q % a.row_tiles;
+        w.skip = it >= n_items;
     }
+    if (w.skip) return w;
     const int* items = a.wl + kWlHead + 2 * a.B;
     w.b = load_uniform(items + 2 * it);
     const int c = load_uniform(items + 2 * it + 1);
@@ -2742,6 +2755,19 @@ bool flash_ctx16_ok(const FlashProblem& p, const FlashPlan& f) {
            (k == Flash16::kCodeRing || k == Flash16::kSpecPv64);
 }
 
+// Whether the row tiles are dealt over the XCDs longest first (spread_tile): from 32
+// row tiles a batch (at least four per XCD, so the tiles on one XCD still share a batch's
+// keys in its L2), for an unsplit causal pass and for any work list.  Below that, verify
+// batches of a few queries keep a batch's tiles on one XCD: their key counts differ by a
+// few keys, and eight XCDs reading every cache would cost more than the balance gains.
+// bf16, with 3d, contiguous tiles against these: causal B = 1, Sq = Sk = 4096 3,746 against
+// 2,320 us; a paged chunk of four sequences' 333 queries over up to 2,011 keys, with its
+// projections, 2,525 against 1,878 us; fp32 B = 8, Sq = Sk = 512 (one batch per XCD either
+// way) 2,528 us in both.
+static bool flash_spread(const FlashProblem& p, const FlashPlan& f) {
+    return f.row_tiles >= 32 && (f.balanced || (p.causal && f.n_split == 1));
+}
+
 hipError_t launch_flash(const FlashProblem& p, const FlashPlan& f, float* ctx, float* row_sum,
                         float* partials, hipStream_t stream, bool merge, void* ctx16) {
     if (ctx16 && !flash_ctx16_ok(p, f)) return hipErrorInvalidValue;
@@ -2799,6 +2825,7 @@ hipError_t launch_flash(const FlashProblem& p, const FlashPlan& f, float* ctx, f
         a.o_scale = p.kv_scale;
     }
     a.causal = p.causal ? 1 : 0;
+    a.spread = flash_spread(p, f) ? 1 : 0;
     a.seq_lens = p.seq_lens;
     a.block_table = p.block_table;
     a.page_size = p.page_size;

@@ -157,6 +157,29 @@ MLA_HD int wl_thread_first(int tid, int B) {
     return wl_min(B, tid * per);
 }
 
+// Order of the row tiles of `units` batches or list items with many tiles each: workgroup p
+// (on XCD p % 8) takes row tile *rt of unit *unit; false past the last one.  Contiguous runs
+// per XCD leave XCDs idle: a causal tile's keys grow with its queries' positions, so with
+// one batch and Sq = Sk the last XCD gets 15/16 of the keys per tile where the mean is 1/2,
+// and a list of four items with one XCD each runs on four.  So units go in groups of eight,
+// one XCD per unit, and the tiles of the last, partial group round-robin over all XCDs; in
+// both the last tiles (the most visible keys) go first, so that the grid ends with short
+// tiles.
+MLA_HD bool spread_tile(int p, int units, int row_tiles, int* unit, int* rt) {
+    const int whole = units / kNumXCDs * kNumXCDs;
+    if (p < whole * row_tiles) {
+        const int q = p / kNumXCDs;
+        *unit = q / row_tiles * kNumXCDs + p % kNumXCDs;
+        *rt = row_tiles - 1 - q % row_tiles;
+        return true;
+    }
+    const int left = units - whole, q = p - whole * row_tiles;
+    if (left == 0 || q >= left * row_tiles) return false;
+    *unit = whole + q % left;
+    *rt = row_tiles - 1 - q / left;
+    return true;
+}
+
 // The list in one thread, batch by batch, with the functions above (the device builder's
 // order among last chunks of one bucket is its LDS atomics'; here it is batch order).
 // Returns the item count.

@@ -130,3 +130,20 @@ def test_dense_splits_fit_one_round_of_cus():
                 assert kps % bk == 0 and kps >= bk
                 assert base * n_split <= 256, (bk, base, Sk, n_split)
                 assert n_split <= max(1, 256 // base), (bk, base, Sk, n_split)
+
+
+@pytest.mark.parametrize("units", [1, 2, 3, 7, 8, 9, 16, 61])
+@pytest.mark.parametrize("row_tiles", [32, 33, 86, 666])
+def test_spread_tiles_cover_once_and_balance(units, row_tiles):
+    """spread_tile deals every row tile of every unit exactly once, nothing past the last,
+    and with causal work (tile rt costs rt + 1) no XCD's share passes the mean by more than
+    one longest tile for every whole group and the partial one."""
+    lib = W.harness()
+    n = units * row_tiles
+    got = [lib.wl_harness_spread_tile(p, units, row_tiles) for p in range(n + 50)]
+    assert sorted(got[:n]) == list(range(n))
+    assert got[n:] == [-1] * 50
+    work = np.zeros(8)
+    for p, t in enumerate(got[:n]):
+        work[p % 8] += t % row_tiles + 1
+    assert work.max() <= work.mean() + row_tiles * (units / 8 + 1) / 8 + row_tiles

@@ -53,6 +53,7 @@ def harness():
               "wl_harness_thread_first"):
         getattr(lib, f).argtypes = [ctypes.c_int, ctypes.c_int]
     lib.wl_harness_dense_keys.argtypes = [ctypes.c_int] * 3
+    lib.wl_harness_spread_tile.argtypes = [ctypes.c_int] * 3
     _LIB = lib
     return lib
 

@@ -20,6 +20,12 @@ int wl_harness_build(const int* seq_lens, int B, int Sk, int row_tiles, int bloc
 
 int wl_harness_bucket(int L, int chunk) { return mla::wl_bucket(L, chunk); }
 
+// -1 past the last tile, else unit * row_tiles + row tile
+int wl_harness_spread_tile(int p, int units, int row_tiles) {
+    int unit, rt;
+    return mla::spread_tile(p, units, row_tiles, &unit, &rt) ? unit * row_tiles + rt : -1;
+}
+
 int wl_harness_thread_first(int tid, int B) { return mla::wl_thread_first(tid, B); }
 
 }
