@@ -303,9 +303,8 @@ struct QLayout {
 bool qup_fused(mla_dtype_t dt, const mla_dims_t* d, const GemmPlan& up) {
     const char* env = getenv("MLA_QUP_FUSE");
     if (env && strcmp(env, "0") == 0) return false;
-    return is_half(dt) && up.wgemm && up.split == 1 && up.bn <= 128 && d->nope % 32 == 0 &&
-           d->rope % 32 == 0 &&
-           d->rope > 0 && d->rope <= 64;
+    return is_half(dt) && (up.bgemm || (up.wgemm && up.bn <= 128)) && up.split == 1 &&
+           d->nope % 32 == 0 && d->rope % 32 == 0 && d->rope > 0 && d->rope <= 64;
 }
 
 // 2a2's fused epilogue with 2c as well (wgemm.hip, qup_supported): one head's nope columns
@@ -314,7 +313,7 @@ bool qup_fused(mla_dtype_t dt, const mla_dims_t* d, const GemmPlan& up) {
 bool qup_fused_2c(mla_dtype_t dt, const mla_dims_t* d, const GemmPlan& up) {
     const char* env = getenv("MLA_QUP_ABSORB");
     if (env && strcmp(env, "0") == 0) return false;
-    return qup_fused(dt, d, up) && up.bn == 128 && up.stages == 4 && d->nope == 128 &&
+    return qup_fused(dt, d, up) && up.wgemm && up.bn == 128 && up.stages == 4 && d->nope == 128 &&
            d->rope == 64 && d->heads % 2 == 0 && d->kv_rank % 128 == 0 && d->kv_rank <= 512;
 }
 

@@ -27,6 +27,7 @@
 #include "kernels.h"
 
 #include <algorithm>
+#include <cmath>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -666,13 +667,9 @@ constexpr TunedPlan kTuned[] = {
     {128, 128, 512, 128, true, false, 64, 64, 1},
     {128, 7168, 16384, 1, false, false, 128, 32, 8},
     {128, 576, 7168, 1, false, false, 64, 64, 8},
-    // B = 128 decode, bf16
-    {128, 1536, 7168, 1, false, true, 128, 64, 8},
-    {128, 24576, 1536, 1, false, true, 128, 96, 1},
+    // B = 128 decode, 16-bit with fp32 A: 2c from q_raw, 3d from ctx and row_sum
     {128, 512, 128, 128, false, true, 128, 128, 1},
     {128, 128, 512, 128, true, true, 32, 128, 1},
-    {128, 7168, 16384, 1, false, true, 128, 128, 8},
-    {128, 576, 7168, 1, false, true, 64, 64, 8},
     // B = 1, 8, 32 decode, fp32: 2a1, 2a2, 2c, 3d
     {1, 1536, 7168, 1, false, false, 32, 128, 16},
     {1, 24576, 1536, 1, false, false, 32, 128, 4},
@@ -728,52 +725,144 @@ bool plan_override(const GemmProblem& p, GemmPlan* out) {
     return false;
 }
 
-// Weight-streaming plans (wgemm.hip), exact shapes: 16-bit products whose weight operand
-// dominates the traffic.  MLA_WGEMM=0 turns the engine off (every shape goes to the tiled
-// engine); MLA_WGEMM_PLAN="M,N,K,G=bn,split[,stages];..." forces a weight-streaming plan for a
-// matching problem (tuning aid, same validity checks).
-struct WTunedPlan { int M, N, K, G; bool nt; int bn, split, stages; };
-constexpr WTunedPlan kWTuned[] = {
-    // B = 128 decode, bf16 / fp16: 2a1, 2a2, and the output projection beside the layer
-    // (63 -> 52 us; the KV projection gained nothing and stays tiled)
-    {128, 1536, 7168, 1, false, 64, 8, 4},
-    {128, 24576, 1536, 1, false, 128, 1, 4},
-    {128, 7168, 16384, 1, false, 128, 4, 4},
-    // 3d from the normalised 16-bit ctx (NT, G = heads): 256 workgroups of 64 columns, the
-    // bf16 attention with 3d 172.4-173.1 us against 174.2-175.7 us on the tiled engine
-    {128, 128, 512, 128, true, 64, 1, 4},
-};
+// The 16-bit products with 16-bit A run on two engines: up to 128 rows on the weight-streaming
+// one (wgemm.hip), past that on the large-tile one (bgemm.hip).  The line lies at one row tile
+// of the former: at M = 160 and 200 its second, nearly empty tile already costs what a full
+// one does (o_proj 98 us at M = 256 against 84-90 on the large tiles at M = 160-200), at
+// M <= 128 it is the faster one for all four weight shapes (o_proj 44-58 against 45-71 us).
+// MLA_WGEMM=0 turns both off (every shape goes to the tiled engine).  MLA_WGEMM_PLAN=
+// "M,N,K,G=bn,split[,stages];..." and MLA_BGEMM_PLAN="M,N,K,G=bm,bn,split;..." force a plan
+// of one engine for a matching problem (tuning aids, same validity checks).
+constexpr int kStreamRows = 128;
 
-bool wgemm_plan(const GemmProblem& p, GemmPlan* out) {
+bool wgemm_off() {
     const char* off = getenv("MLA_WGEMM");
-    if (off && strcmp(off, "0") == 0) return false;
-    int bn = 0, split = 0, stages = 4;
-    if (const char* env = getenv("MLA_WGEMM_PLAN")) {
-        const char* s = env;
-        while (*s && !bn) {
-            long M, N, K, G;
-            int b, sp, used = 0, used2 = 0, ns = 4;
-            if (sscanf(s, "%ld,%ld,%ld,%ld=%d,%d%n", &M, &N, &K, &G, &b, &sp, &used) != 6) break;
-            if (sscanf(s + used, ",%d%n", &ns, &used2) == 1) used += used2;
-            if (M == p.M && N == p.N && K == p.K && G == p.G) { bn = b; split = sp; stages = ns; }
-            s += used;
-            while (*s == ';' || *s == ' ') ++s;
+    return off && strcmp(off, "0") == 0;
+}
+
+bool bgemm_forced(const GemmProblem& p, GemmPlan* out) {
+    const char* s = getenv("MLA_BGEMM_PLAN");
+    while (s && *s) {
+        long M, N, K, G;
+        int bm, bn, split, used = 0;
+        if (sscanf(s, "%ld,%ld,%ld,%ld=%d,%d,%d%n", &M, &N, &K, &G, &bm, &bn, &split, &used) != 7) break;
+        if (M == p.M && N == p.N && K == p.K && G == p.G) {
+            if (!bgemm_supported(p, bm, bn, split)) return false;
+            out->bm = bm; out->bn = bn; out->split = split; out->tiles_per_wg = 1; out->bgemm = true;
+            return true;
         }
+        s += used;
+        while (*s == ';' || *s == ' ') ++s;
     }
-    for (const auto& t : kWTuned)
-        if (!bn && t.M == p.M && t.N == p.N && t.K == p.K && t.G == p.G && t.nt == p.b_nt) {
-            bn = t.bn; split = t.split; stages = t.stages;
-        }
+    return false;
+}
+
+bool wgemm_runs(const GemmProblem& p, int bn, int split, int stages) {
     const bool ring_ok = (bn == 256 && stages == 3 && !p.b_nt) ||
                          (bn == 128 && (stages == 3 || stages == 4)) ||
                          (bn == 64 && (stages == 3 || stages == 4 || (stages == 6 && !p.b_nt)));
-    if (!bn || split < 1 || !ring_ok || !wgemm_supported(p, bn, split)) return false;
+    if (split < 1 || !ring_ok || !wgemm_supported(p, bn, split)) return false;
     const int kslices = cdiv(p.K, 64);
-    const int per = cdiv(kslices, std::min(split, kslices));
-    if (!wgemm_supported(p, bn, cdiv(kslices, per))) return false;
+    return wgemm_supported(p, bn, cdiv(kslices, cdiv(kslices, std::min(split, kslices))));
+}
+
+void wgemm_set(GemmPlan* out, int bn, int split, int stages) {
     out->bm = 128; out->bn = bn; out->split = split; out->tiles_per_wg = 1; out->wgemm = true;
     out->stages = stages;
-    return true;
+}
+
+bool wgemm_forced(const GemmProblem& p, GemmPlan* out) {
+    const char* s = getenv("MLA_WGEMM_PLAN");
+    while (s && *s) {
+        long M, N, K, G;
+        int bn, split, used = 0, used2 = 0, stages = 4;
+        if (sscanf(s, "%ld,%ld,%ld,%ld=%d,%d%n", &M, &N, &K, &G, &bn, &split, &used) != 6) break;
+        if (sscanf(s + used, ",%d%n", &stages, &used2) == 1) used += used2;
+        if (M == p.M && N == p.N && K == p.K && G == p.G) {
+            if (!wgemm_runs(p, bn, split, stages)) return false;
+            wgemm_set(out, bn, split, stages);
+            return true;
+        }
+        s += used;
+        while (*s == ';' || *s == ' ') ++s;
+    }
+    return false;
+}
+
+// Splits of the 64-deep K slices without an empty one, up to 16: past that the consumer's sum
+// over the partials costs more than the shorter loops give.
+constexpr int kMaxSplit = 16;
+bool whole_split(int kslices, int split, int* per) {
+    *per = cdiv(kslices, split);
+    return cdiv(kslices, *per) == split;
+}
+
+// Weight streaming, M <= 128: the time is the weights' stream or the slices of one workgroup,
+// whichever is longer, plus the split partials and their sum.  Measured (flushed weights):
+// 0.27 us a 64-deep slice on 64 columns, 0.5 on 128; the stream reaches 5.3 TB/s in rows of
+// 256 bytes and 3.9 in rows of 128 (64 columns, NN), from about 192 workgroups up.  It gives
+// 2a1 64 columns x 8 splits (12.2-15.8 us for M = 1..128 against 17.2-21.9 on the tiled
+// engine), 2a2 128 x 1 (17-22 / 31-37), o_proj 128 x 4 (44-58 / 107-117), the KV projection
+// 64 x 14 (11.4-13.7 / 14.1-16.4), 3d at M = 128 64 columns (172.4-173.1 us with the
+// attention against 174.2-175.7).
+bool wgemm_rule(const GemmProblem& p, GemmPlan* out) {
+    if (p.M > kStreamRows) return false;
+    const int kslices = cdiv(p.K, 64);
+    double best = 1e300;
+    for (int bn : {128, 64})
+        for (int split = 1; split <= std::min(kMaxSplit, kslices); ++split) {
+            int per;
+            if (!whole_split(kslices, split, &per) || !wgemm_runs(p, bn, split, 4)) continue;
+            const double wgs = (double)(p.N / bn) * p.G * split;
+            const double rounds = std::ceil(wgs / kNumCUs);
+            const double rate = (bn == 64 && !p.b_nt ? 3.9e6 : 5.3e6) * std::min(1.0, wgs / 192);
+            const double bytes = 2.0 * p.K * p.N * p.G;
+            double t = std::max(rounds * per * (bn == 64 ? 0.27 : 0.5), bytes / rate);
+            if (split > 1) t += 1.5 + 0.2 * split + 4.0 * (split + 1) * p.M * p.N * p.G / 3.7e6;
+            if (t < best * 0.999) {
+                best = t;
+                wgemm_set(out, bn, split, 4);
+            }
+        }
+    return best < 1e300;
+}
+
+// Large tiles, M > 128.  A workgroup's time is its 32-deep slices at the tile's slice time --
+// of a lightly loaded chip, and what a full one adds as its clock drops -- plus ~5.6 us of
+// launch, first loads and stores; rounds of 256 workgroups (128 x 128: two per CU, where one's
+// stores pass under the other's MFMAs: 4 us).  Fitted to 500 measured (shape, plan) pairs of
+// the four weight products at M = 160..4096 (9% rms; the plan it picks is within 10% of the
+// best measured one everywhere, and the best at most).  3d (N = 128, K = 512) takes 128 x 128
+// (M = 4096: 188 against 214 us on 256 x 128), 2c (K = 128) 256 x 256 (M = 2048: 111-116
+// against 157 on 256 x 128 and 129 on 128 x 128).
+bool bgemm_rule(const GemmProblem& p, GemmPlan* out) {
+    if (p.M <= kStreamRows) return false;
+    struct Tile { int bm, bn, per_cu; double slice, load, fixed; };   // us
+    constexpr Tile kBTiles[] = {{256, 256, 1, 0.56, 0.25, 5.6}, {256, 128, 1, 0.40, 0.14, 5.6},
+                                {128, 128, 2, 0.19, 0.21, 4.0}};
+    const int kslices = cdiv(p.K, 64);
+    double best = 1e300;
+    for (const Tile& b : kBTiles)
+        for (int split = 1; split <= std::min(kMaxSplit, kslices); ++split) {
+            int per;
+            if (!whole_split(kslices, split, &per) || !bgemm_supported(p, b.bm, b.bn, split)) continue;
+            const double nsl = 2.0 * per;
+            const int64_t wgs = (int64_t)cdiv(p.M, b.bm) * cdiv(p.N, b.bn) * p.G * split;
+            const int64_t cap = (int64_t)kNumCUs * b.per_cu, left = wgs % cap;
+            double t = (double)(wgs / cap) * (nsl * (b.per_cu * b.slice + b.load) + b.fixed);
+            if (left)
+                t += nsl * ((left > kNumCUs ? b.per_cu : 1) * b.slice + b.load * left / cap) + b.fixed;
+            const double bytes = (2.0 * p.K * p.N + 2.0 * p.M * p.K +
+                                  (p.out_type == kOutF32 ? 4.0 : 2.0) * p.M * p.N) * p.G;
+            t = std::max(t, bytes / 5.9e6 + b.fixed);
+            if (split > 1) t += 4.0 * (split + 1) * p.M * p.N * p.G / 3.7e6;
+            if (t < best * 0.999) {
+                best = t;
+                out->bm = b.bm; out->bn = b.bn; out->split = split; out->tiles_per_wg = 1;
+                out->bgemm = true;
+            }
+        }
+    return best < 1e300;
 }
 
 }  // namespace
@@ -789,7 +878,10 @@ GemmPlan plan_gemm(const GemmProblem& p) {
     const int kslices = cdiv(p.K, kBK);
     GemmPlan best;
     double best_t = 1e300;
-    if (!wgemm_plan(p, &best) && !plan_override(p, &best) && !tuned_plan(p, &best)) {
+    const bool half_rules = !wgemm_off();
+    if (!(half_rules && (bgemm_forced(p, &best) || wgemm_forced(p, &best))) &&
+        !plan_override(p, &best) &&
+        !(half_rules && (wgemm_rule(p, &best) || bgemm_rule(p, &best))) && !tuned_plan(p, &best)) {
         for (const auto& t : kTiles) {
             const int tm = cdiv(p.M, t.bm), tn = cdiv(p.N, t.bn);
             const int64_t tiles = (int64_t)tm * tn * p.G;
@@ -853,8 +945,9 @@ hipError_t split_reduce(const GemmProblem& p, const GemmArgs& a, int split, hipS
 hipError_t launch_gemm_impl(const GemmProblem& p, const GemmPlan& plan, void* workspace,
                             bool reduce, hipStream_t stream) {
     // the epilogue addresses a tile's rows with 32-bit offsets from the tile's first row
+    // (the large-tile engine's with 64-bit ones)
     const int64_t out_ld = plan.split > 1 ? p.N : p.ldc;
-    if ((int64_t)plan.bm * out_ld * 4 >= (int64_t)kRsrcRange) return hipErrorInvalidValue;
+    if (!plan.bgemm && (int64_t)plan.bm * out_ld * 4 >= (int64_t)kRsrcRange) return hipErrorInvalidValue;
     GemmArgs a;
     a.A = p.A; a.lda = p.lda; a.sAg = p.sAg;
     a.B = p.B; a.ldb = p.ldb; a.sBg = p.sBg;
@@ -897,6 +990,11 @@ hipError_t launch_gemm_impl(const GemmProblem& p, const GemmPlan& plan, void* wo
         return hipErrorInvalidValue;
     const int64_t nblocks64 = (int64_t)a.tiles_m * a.tiles_n * a.G * a.split;
     if (nblocks64 <= 0 || nblocks64 > 0x7fffffff) return hipErrorInvalidValue;
+    if (plan.bgemm && bgemm_aligned(p)) {
+        const hipError_t e = launch_bgemm(p, plan, a.ws, stream);
+        if (e != hipSuccess || plan.split == 1 || !reduce) return e;
+        return split_reduce(p, a, plan.split, stream);
+    }
     if (p.qup && !(plan.wgemm && wgemm_aligned(p))) return hipErrorInvalidValue;
     if (plan.wgemm && wgemm_aligned(p)) {
         const hipError_t e = launch_wgemm(p, plan, a.ws, stream);

@@ -82,6 +82,7 @@ struct GemmPlan {
     int tiles_per_wg = 1;     // > 1: persistent grid of ceil(tiles / tiles_per_wg) workgroups
     size_t workspace_bytes = 0;  // fp32 partials when split > 1
     bool wgemm = false;       // the weight-streaming engine (wgemm.hip): bm 128, bn 64 / 128
+    bool bgemm = false;       // the large-tile engine (bgemm.hip): 256x256, 256x128, 128x128
     int stages = 4;           // its LDS ring depth
 };
 
@@ -97,6 +98,12 @@ bool wgemm_supported(const GemmProblem& p, int bn, int split);
 bool qup_supported(const GemmProblem& p, const QUpEpilogue& q, const GemmPlan& plan);
 bool wgemm_aligned(const GemmProblem& p);
 hipError_t launch_wgemm(const GemmProblem& p, const GemmPlan& plan, float* partials,
+                        hipStream_t stream);
+// Large-tile engine: 16-bit A and B, NN or NT, plain A, N % 8 == 0, K % 32 == 0, outputs as
+// above (a 16-bit C in rows of 16 bytes).  bgemm_aligned: the pointers' side, as above.
+bool bgemm_supported(const GemmProblem& p, int bm, int bn, int split);
+bool bgemm_aligned(const GemmProblem& p);
+hipError_t launch_bgemm(const GemmProblem& p, const GemmPlan& plan, float* partials,
                         hipStream_t stream);
 hipError_t launch_gemm(const GemmProblem& p, const GemmPlan& plan, void* workspace,
                        hipStream_t stream);

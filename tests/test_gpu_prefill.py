@@ -1,6 +1,6 @@
 """GPU parity of prefill-sized calls (many query tokens per sequence) against the float64
 oracle: the orders in which row tiles are dealt over the XCDs, on the dense and the paged
-pass.  Tolerances are the parity tests' own (attn_cases.tol)."""
+pass, and the 16-bit products on both engines.  Tolerances are the parity tests' own (attn_cases.tol)."""
 
 from __future__ import annotations
 
@@ -67,3 +67,81 @@ def test_paged_row_tiles_over_xcds(ext, dt, lens):
         ref = R.mla_attention_paged(qa.double(), qr.double(), ck.double(), pe.double(), table, sl,
                                     wuv.double(), SCALE, causal=causal).float()
         torch.testing.assert_close(got, ref, **C.tol(dt, ref))
+
+
+# ---- the large-tile GEMM engine
+
+def gemm_inputs(M, N, K, dt):
+    g = torch.Generator().manual_seed(M + N + K)
+    A = torch.randn(M, K, generator=g).to(dt)
+    W = (torch.randn(K, N, generator=g) / math.sqrt(K)).to(dt)
+    return A, W
+
+
+@pytest.mark.parametrize("dt", [BF, H16], ids=["bf16", "f16"])
+@pytest.mark.parametrize("M,N,K,plan", [
+    (256, 256, 1024, "256,256,1"),   # one whole tile
+    (257, 264, 96, "256,256,1"),     # a row and a chunk of columns past it, fewer slices than stages
+    (40, 200, 32, "256,128,1"),      # one slice, rows and columns off the tile
+    (700, 576, 416, "256,128,3"),    # slices 6, 6, 1 of 32 over the splits
+    (1332, 1536, 512, "128,128,2"),  # many row tiles, the last of 52 rows
+    (130, 392, 224, "128,128,1"),
+    (2100, 512, 64, "256,256,1"),    # past one group of eight row tiles
+])
+def test_large_tile_gemm(ext, monkeypatch, dt, M, N, K, plan):
+    """Forced large-tile plans against the float64 product of the same 16-bit values (fp32
+    sums of K terms of unit total variance: 1e-4 as for the other engines)."""
+    A, W = gemm_inputs(M, N, K, dt)
+    monkeypatch.setenv("MLA_BGEMM_PLAN", f"{M},{N},{K},1={plan}")
+    got = ext.gemm(gpu(A), gpu(W)).cpu()
+    ref = (A.double() @ W.double()).float()
+    torch.testing.assert_close(got, ref, rtol=1e-4, atol=1e-4)
+
+
+@pytest.mark.parametrize("M", [1, 100, 128, 129, 300, 520])
+@pytest.mark.parametrize("N,K", [(576, 7168), (1536, 640), (200, 192)])
+def test_16bit_products_by_rule(ext, M, N, K):
+    """The plans that the rules pick on both sides of the engines' line (128 rows), among
+    them columns that only the large tiles take, against float64 (see above)."""
+    A, W = gemm_inputs(M, N, K, BF)
+    got = ext.gemm(gpu(A), gpu(W)).cpu()
+    torch.testing.assert_close(got, (A.double() @ W.double()).float(), rtol=1e-4, atol=1e-4)
+
+
+@pytest.mark.parametrize("dt", [BF, H16], ids=["bf16", "f16"])
+@pytest.mark.parametrize("B,Sq,per_seq", [(5, 26, True), (3, 87, False), (150, 2, True)])
+def test_q_absorbed_many_rows(ext, monkeypatch, dt, B, Sq, per_seq):
+    """2a2 on the large tiles with 2b in its epilogue, and 2c from its 16-bit q_nope on them:
+    the same bits as 2a2, the 2b launch and 2c on the tiled engine from fp32 q_raw
+    (MLA_QUP_FUSE=0: the same 2a1 and 2a2 sums), and the fp32 oracle's result."""
+    inp = R.make_inputs(B, Sq, max(Sq, 64), seed=B + Sq, dtype=dt)
+    W_uk, _ = R.split_wkv_b(inp["wkv_b"], D.nope)
+    pos = inp["positions"]
+    if per_seq:
+        pos = torch.arange(Sq)[None] + 4900 - 31 * torch.arange(B)[:, None]
+    args = [gpu(inp[k]) for k in ("x", "W_q_a", "q_norm_w", "W_q_b")] + [gpu(W_uk.contiguous()),
+                                                                        gpu(pos)]
+    qa, qr = (t.cpu() for t in ext.q_absorbed(*args, D.nope, D.rope, 1e-6))
+    monkeypatch.setenv("MLA_QUP_FUSE", "0")
+    qa0, qr0 = (t.cpu() for t in ext.q_absorbed(*args, D.nope, D.rope, 1e-6))
+    assert torch.equal(qa, qa0) and torch.equal(qr, qr0)
+    f = {k: inp[k].float() for k in ("x", "W_q_a", "q_norm_w", "W_q_b")}
+    pick = [0, B // 2, B - 1]
+    if per_seq:
+        ra, rr = R.prepare_q_ragged(f["x"][pick], f["W_q_a"], f["q_norm_w"], f["W_q_b"],
+                                    W_uk.float(), pos[pick], D.nope, D.rope)
+    else:
+        ra, rr = R.prepare_q_mla_absorbed(f["x"][pick], f["W_q_a"], f["q_norm_w"], f["W_q_b"],
+                                          W_uk.float(), pos, D.nope, D.rope)
+    torch.testing.assert_close(qa[pick].float(), ra, **C.tol(dt, ra))
+    torch.testing.assert_close(qr[pick].float(), rr, **C.tol(dt, rr))
+
+
+@pytest.mark.parametrize("dt", [BF, H16], ids=["bf16", "f16"])
+@pytest.mark.parametrize("B,Sq", [(260, 1), (2, 130), (300, 2)])
+def test_out_projection_many_rows(ext, monkeypatch, dt, B, Sq):
+    """3d on the large tiles (NT, G = heads) gives the tiled engine's bits (MLA_WGEMM=0)."""
+    args = [gpu(t) for t in C.attn_inputs(B, Sq, 140, seed=B, dt=dt)]
+    got = ext.mla_attention(*args, SCALE, Sq > 1).cpu()
+    monkeypatch.setenv("MLA_WGEMM", "0")
+    assert torch.equal(got, ext.mla_attention(*args, SCALE, Sq > 1).cpu())
