@@ -1510,9 +1510,11 @@ int mla_attention_paged_fp8kv(mla_dtype_t dtype, const mla_dims_t* dims, const v
     fp.seq_lens = seq_lens;
     fp.block_table = block_table;
     fp.page_size = page_size;
-    MLA_TRY_HIP(launch_flash(fp, L.flash, ctx, row_sum, at<float>(workspace, L.off_part), stream),
+    MLA_TRY_HIP(launch_flash(fp, L.flash, ctx, row_sum, at<float>(workspace, L.off_part), stream,
+                             true, L.ctx16 ? ctx : nullptr),
                 "paged fp8-cache attention launch");
-    GemmProblem op = out_problem(MLA_DTYPE_BF16, dims, ctx, row_sum, W_uv, out);
+    GemmProblem op = L.ctx16 ? out_problem16(MLA_DTYPE_BF16, dims, ctx, W_uv, out)
+                             : out_problem(MLA_DTYPE_BF16, dims, ctx, row_sum, W_uv, out);
     MLA_TRY_HIP(launch_gemm(op, L.out, at<void>(workspace, L.off_out_ws), stream), "3d launch");
     return ok();
 }
@@ -1721,9 +1723,11 @@ int mla_attention_paged(mla_dtype_t dtype, const mla_dims_t* dims, const void* q
                         "3d launch");
             return ok();
         }
-        MLA_TRY_HIP(launch_flash(fp, L.flash, ctx, row_sum, part, stream),
+        MLA_TRY_HIP(launch_flash(fp, L.flash, ctx, row_sum, part, stream, true,
+                                 L.ctx16 ? ctx : nullptr),
                     "fused paged attention launch");
-        GemmProblem op = out_problem(dtype, dims, ctx, row_sum, W_uv, out);
+        GemmProblem op = L.ctx16 ? out_problem16(dtype, dims, ctx, W_uv, out)
+                                 : out_problem(dtype, dims, ctx, row_sum, W_uv, out);
         MLA_TRY_HIP(launch_gemm(op, L.out, at<void>(workspace, L.off_out_ws), stream),
                     "3d launch");
         return ok();

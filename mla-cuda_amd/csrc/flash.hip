@@ -80,7 +80,8 @@ struct FlashArgs {
     float* o_direct;
     float* l_direct;
     int spread;        // deal the row tiles over the XCDs, longest first (flash_spread)
-    // dense unsplit 16-bit pass only (flash_ctx16_ok): instead of o / l, write each row
+    // 16-bit passes only (flash_ctx16_ok): instead of ctx / row_sum (an unsplit pass's o / l,
+    // a list's o_direct / l_direct), write each row
     // already normalised and rounded to the storage format, (o_scale O) (1 / l) -- what
     // 3d's A staging forms from ctx and row_sum -- at ctx16[row][R]
     void* ctx16;
@@ -1120,7 +1121,7 @@ __global__ void __launch_bounds__(kXThreads, 1) flash16x_kernel(FlashArgs a) {
             const float lsum = xlr[l32] + xlr[32 + l32];
             const float M = xref[t * 64 + l32];
             const int64_t slot = (work.direct ? (int64_t)b : work.slot) * rows_b + row;
-            if (a.ctx16) {
+            if (a.ctx16 && (work.direct || (!a.wl && a.n_split == 1))) {
                 const float r = lsum == 0.f ? 0.f : 1.f / lsum;
                 uint16_t* crow = static_cast<uint16_t*>(a.ctx16) + slot * kFR + 128 * cq + 4 * hw;
                 #pragma unroll
@@ -1527,7 +1528,7 @@ __global__ void __launch_bounds__(kXThreads, 1) flash16x8_kernel(FlashArgs a) {
         const float lsum = xlr[l32] + xlr[32 + l32];
         const float M = xref[t * 64 + l32];
         const int64_t slot = (work.direct ? (int64_t)b : work.slot) * rows_b + row;
-        if (a.ctx16) {
+        if (a.ctx16 && (work.direct || (!a.wl && a.n_split == 1))) {
             const float r = lsum == 0.f ? 0.f : 1.f / lsum;
             uint16_t* crow = static_cast<uint16_t*>(a.ctx16) + slot * kFR + 128 * cq + 4 * hw;
             #pragma unroll
@@ -2413,69 +2414,132 @@ __global__ void __launch_bounds__(kFThreads, 1) flash32w_kernel(FlashArgs a) {
 
 constexpr int kFStages = 4;   // LDS ring depth
 
-// ctx = sum_s w_s O_s, row_sum = sum_s w_s l_s, w_s = 2^(m_s - max_s m_s).  One workgroup
-// per row: its threads take the row maximum over the splits, then wave w sums splits
-// w, w+4, ... (lane: 8 columns), and the four waves' sums are added in wave order -- a
-// fixed order, so the merge is deterministic.  Each wave keeps a split's 2 KB row in
-// flight per iteration, so many splits (small batches) do not serialise on latency.
-// Split s of row r (batch b, row i of the batch) is partial slot unit(s) * rows_b + i:
-// unit(s) = s * B + b for the uniform splits, first[b] + s for a work list (whose batches
-// of one chunk were written straight to ctx / row_sum and are skipped here).
+// ctx = sum_s w_s O_s, row_sum = sum_s w_s l_s, w_s = 2^(m_s - max_s m_s), written as fp32 ctx
+// and row_sum, or (OUT 16-bit) normalised and rounded to the storage format as the unsplit
+// passes do.  Split s of row r (batch b, row i of the batch) is partial slot
+// unit(s) * rows_b + i: unit(s) = s * B + b for the uniform splits, first[b] + s for a work
+// list (whose batches of one chunk were written directly and are skipped here).
+//
+// It is bound by the partial rows' bytes (2 KB each), if enough of them are in flight:
+//   up to kMergeFew splits a wave sums a row (lane: 8 columns), all its loads going out
+//     together, and a workgroup takes rows_per_wg rows, four at a time;
+//   past that the four waves share a row: the threads take its maximum, wave w sums splits
+//     w, w + 4, ... and the four sums are added in wave order.  Small batches, which have
+//     many splits and few rows, get one row per workgroup.
+// Both orders are fixed, so the merge is deterministic.  The rows of a single-chunk batch cost
+// one list read per workgroup: one workgroup per row took 45 us to find the 170,496 rows of a
+// prefill chunk's four sequences already written.
+constexpr int kMergeFew = 8;
+template <int OUT>
 __global__ void __launch_bounds__(256) flash_merge_kernel(const float* __restrict__ o,
                                                           const float* __restrict__ m,
                                                           const float* __restrict__ l,
-                                                          float* __restrict__ ctx,
+                                                          void* __restrict__ ctx,
                                                           float* __restrict__ row_sum, int B,
-                                                          int rows_b, int n_split,
+                                                          int rows, int rows_b, int n_uniform,
+                                                          int rows_per_wg,
                                                           const int* __restrict__ wl) {
     __shared__ float red[256];
     __shared__ v4f part[4][64][2];
     __shared__ float lpart[4];
-    const int r = blockIdx.x, tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-    const int b = r / rows_b, i = r - b * rows_b;
-    int64_t unit0 = b, unit_step = B;
-    if (wl) {
-        n_split = load_uniform(wl + kWlHead + B + b);
-        if (n_split == 1) return;
-        unit0 = load_uniform(wl + kWlHead + b);
-        unit_step = 1;
-    }
-    auto slot_of = [&](int s) { return (unit0 + s * unit_step) * rows_b + i; };
-    float mx = -INFINITY;
-    for (int s = tid; s < n_split; s += 256) mx = fmaxf(mx, m[slot_of(s)]);
-    red[tid] = mx;
-    __syncthreads();
-    #pragma unroll
-    for (int w = 128; w > 0; w >>= 1) {
-        if (tid < w) red[tid] = fmaxf(red[tid], red[tid + w]);
-        __syncthreads();
-    }
-    mx = red[0];
-    v4f acc0 = {0.f, 0.f, 0.f, 0.f}, acc1 = acc0;
-    float ls = 0.f;
-    for (int s = wave; s < n_split; s += 4) {
-        const int64_t slot = slot_of(s);
-        const float ms = m[slot];
-        const float w = ms == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(ms - mx);
-        const v4f* src = reinterpret_cast<const v4f*>(o + slot * kFR) + 2 * lane;
-        acc0 += w * src[0];
-        acc1 += w * src[1];
-        ls += w * l[slot];
-    }
-    part[wave][lane][0] = acc0;
-    part[wave][lane][1] = acc1;
-    if (lane == 0) lpart[wave] = ls;
-    __syncthreads();
-    if (wave == 0) {
-        #pragma unroll
-        for (int w = 1; w < 4; ++w) {
-            acc0 += part[w][lane][0];
-            acc1 += part[w][lane][1];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    auto splits_of = [&](int r, int64_t* unit0, int64_t* step) __attribute__((always_inline)) {
+        const int b = r / rows_b;
+        *unit0 = wl ? load_uniform(wl + kWlHead + b) : b;
+        *step = wl ? 1 : B;
+        return wl ? load_uniform(wl + kWlHead + B + b) : n_uniform;
+    };
+    auto store = [&](int r, v4f a0, v4f a1, float ls) __attribute__((always_inline)) {
+        if constexpr (OUT == kOutF32) {
+            v4f* dst = reinterpret_cast<v4f*>(static_cast<float*>(ctx) + (int64_t)r * kFR) + 2 * lane;
+            dst[0] = a0;
+            dst[1] = a1;
+            if (lane == 0) row_sum[r] = ls;
+        } else {
+            using S = Store16<OUT>;
+            const float f = ls == 0.f ? 0.f : 1.f / ls;
+            const v4f w0 = a0 * f, w1 = a1 * f;
+            reinterpret_cast<v4u*>(static_cast<uint16_t*>(ctx) + (int64_t)r * kFR)[lane] =
+                v4u{S::pack2(w0[0], w0[1]), S::pack2(w0[2], w0[3]), S::pack2(w1[0], w1[1]),
+                    S::pack2(w1[2], w1[3])};
         }
-        v4f* dst = reinterpret_cast<v4f*>(ctx + (int64_t)r * kFR) + 2 * lane;
-        dst[0] = acc0;
-        dst[1] = acc1;
-        if (lane == 0) row_sum[r] = ((lpart[0] + lpart[1]) + lpart[2]) + lpart[3];
+    };
+    const int r_end = min(rows, ((int)blockIdx.x + 1) * rows_per_wg);
+    for (int r0 = blockIdx.x * rows_per_wg, next; r0 < r_end; r0 = next) {
+        int64_t unit0, step;
+        const int n0 = splits_of(r0, &unit0, &step);
+        if (wl && n0 == 1) {   // on to the next batch
+            next = (r0 / rows_b + 1) * rows_b;
+            continue;
+        }
+        next = r0 + 4;
+        const int last = min(next, r_end) - 1;
+        const bool one_batch = r0 / rows_b == last / rows_b;
+        if (rows_per_wg == 1 || (one_batch && n0 > kMergeFew)) {
+            // the workgroup, row by row
+            for (int r = r0; r <= last; ++r) {
+                const int i = r % rows_b;
+                auto slot_of = [&](int s) { return (unit0 + s * step) * rows_b + i; };
+                float mx = -INFINITY;
+                for (int s = tid; s < n0; s += 256) mx = fmaxf(mx, m[slot_of(s)]);
+                __syncthreads();   // the row before is done with red and part
+                red[tid] = mx;
+                __syncthreads();
+                #pragma unroll
+                for (int w = 128; w > 0; w >>= 1) {
+                    if (tid < w) red[tid] = fmaxf(red[tid], red[tid + w]);
+                    __syncthreads();
+                }
+                mx = red[0];
+                v4f acc0 = {0.f, 0.f, 0.f, 0.f}, acc1 = acc0;
+                float ls = 0.f;
+                for (int s = wave; s < n0; s += 4) {
+                    const int64_t slot = slot_of(s);
+                    const float ms = m[slot];
+                    const float w = ms == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(ms - mx);
+                    const v4f* src = reinterpret_cast<const v4f*>(o + slot * kFR) + 2 * lane;
+                    acc0 += w * src[0];
+                    acc1 += w * src[1];
+                    ls += w * l[slot];
+                }
+                part[wave][lane][0] = acc0;
+                part[wave][lane][1] = acc1;
+                if (lane == 0) lpart[wave] = ls;
+                __syncthreads();
+                if (wave == 0) {
+                    #pragma unroll
+                    for (int w = 1; w < 4; ++w) {
+                        acc0 += part[w][lane][0];
+                        acc1 += part[w][lane][1];
+                    }
+                    store(r, acc0, acc1, ((lpart[0] + lpart[1]) + lpart[2]) + lpart[3]);
+                }
+            }
+            continue;
+        }
+        const int r = r0 + wave;   // a wave's row
+        if (r > last) continue;
+        const int n = splits_of(r, &unit0, &step);
+        if (wl && n == 1) continue;
+        const int i = r % rows_b;
+        auto slot_of = [&](int s) { return (unit0 + s * step) * rows_b + i; };
+        float mx = -INFINITY;
+        for (int s = lane; s < n; s += 64) mx = fmaxf(mx, m[slot_of(s)]);
+        mx = wave_reduce(mx, OpMax{});
+        v4f acc0 = {0.f, 0.f, 0.f, 0.f}, acc1 = acc0;
+        float ls = 0.f;
+        #pragma unroll 4
+        for (int s = 0; s < n; ++s) {
+            const int64_t slot = slot_of(s);
+            const float ms = m[slot];
+            const float w = ms == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(ms - mx);
+            const v4f* src = reinterpret_cast<const v4f*>(o + slot * kFR) + 2 * lane;
+            acc0 += w * src[0];
+            acc1 += w * src[1];
+            ls += w * l[slot];
+        }
+        store(r, acc0, acc1, ls);
     }
 }
 
@@ -2751,7 +2815,7 @@ bool flash_ctx16_ok(const FlashProblem& p, const FlashPlan& f) {
     const char* env = std::getenv("MLA_CTX16");
     if (env && env[0] == '0') return false;
     const Flash16 k = flash16_choice(p);
-    return (p.half || p.fp8_kv) && !f.balanced && !f.wave && f.n_split == 1 &&
+    return (p.half || p.fp8_kv) && !f.wave &&
            (k == Flash16::kCodeRing || k == Flash16::kSpecPv64);
 }
 
@@ -2879,8 +2943,19 @@ hipError_t launch_flash(const FlashProblem& p, const FlashPlan& f, float* ctx, f
     hipError_t e = hipGetLastError();
     if (e != hipSuccess || (!f.balanced && f.n_split == 1)) return e;
     if (!merge && !f.balanced) return e;   // the caller folds the merge in
-    hipLaunchKernelGGL(flash_merge_kernel, dim3((unsigned)rows), dim3(256), 0, stream, a.o,
-                       a.m, a.l, ctx, row_sum, p.B, rows_b, f.n_split, a.wl);
+    // few rows: one per workgroup; many: four, and 64 once that still fills the chip
+    const int rpw = rows <= 2048 ? 1 : rows < 65536 ? 4 : 64;
+    const dim3 mgrid((unsigned)((rows + rpw - 1) / rpw)), mblock(256);
+    const int n = f.n_split;
+    if (!ctx16)
+        hipLaunchKernelGGL(flash_merge_kernel<kOutF32>, mgrid, mblock, 0, stream, a.o, a.m, a.l, ctx,
+                           row_sum, p.B, rows, rows_b, n, rpw, a.wl);
+    else if (p.f16)
+        hipLaunchKernelGGL(flash_merge_kernel<kOutF16>, mgrid, mblock, 0, stream, a.o, a.m, a.l,
+                           ctx16, nullptr, p.B, rows, rows_b, n, rpw, a.wl);
+    else
+        hipLaunchKernelGGL(flash_merge_kernel<kOutBF16>, mgrid, mblock, 0, stream, a.o, a.m, a.l,
+                           ctx16, nullptr, p.B, rows, rows_b, n, rpw, a.wl);
     return hipGetLastError();
 }
 

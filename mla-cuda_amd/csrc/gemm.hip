@@ -790,8 +790,10 @@ bool wgemm_forced(const GemmProblem& p, GemmPlan* out) {
 }
 
 // Splits of the 64-deep K slices without an empty one, up to 16: past that the consumer's sum
-// over the partials costs more than the shorter loops give.
+// over the partials costs more than the shorter loops give.  Grouped products (2c, 3d: K = 128
+// and 512, a group per head) are not split, so they need no workspace.
 constexpr int kMaxSplit = 16;
+int max_split(const GemmProblem& p, int kslices) { return p.G > 1 ? 1 : std::min(kMaxSplit, kslices); }
 bool whole_split(int kslices, int split, int* per) {
     *per = cdiv(kslices, split);
     return cdiv(kslices, *per) == split;
@@ -807,10 +809,10 @@ bool whole_split(int kslices, int split, int* per) {
 // attention against 174.2-175.7).
 bool wgemm_rule(const GemmProblem& p, GemmPlan* out) {
     if (p.M > kStreamRows) return false;
-    const int kslices = cdiv(p.K, 64);
+    const int kslices = cdiv(p.K, 64), most = max_split(p, kslices);
     double best = 1e300;
     for (int bn : {128, 64})
-        for (int split = 1; split <= std::min(kMaxSplit, kslices); ++split) {
+        for (int split = 1; split <= most; ++split) {
             int per;
             if (!whole_split(kslices, split, &per) || !wgemm_runs(p, bn, split, 4)) continue;
             const double wgs = (double)(p.N / bn) * p.G * split;
@@ -840,10 +842,10 @@ bool bgemm_rule(const GemmProblem& p, GemmPlan* out) {
     struct Tile { int bm, bn, per_cu; double slice, load, fixed; };   // us
     constexpr Tile kBTiles[] = {{256, 256, 1, 0.56, 0.25, 5.6}, {256, 128, 1, 0.40, 0.14, 5.6},
                                 {128, 128, 2, 0.19, 0.21, 4.0}};
-    const int kslices = cdiv(p.K, 64);
+    const int kslices = cdiv(p.K, 64), most = max_split(p, kslices);
     double best = 1e300;
     for (const Tile& b : kBTiles)
-        for (int split = 1; split <= std::min(kMaxSplit, kslices); ++split) {
+        for (int split = 1; split <= most; ++split) {
             int per;
             if (!whole_split(kslices, split, &per) || !bgemm_supported(p, b.bm, b.bn, split)) continue;
             const double nsl = 2.0 * per;
