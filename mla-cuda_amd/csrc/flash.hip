@@ -704,6 +704,76 @@ __global__ void __launch_bounds__(kFThreads, 1) flash16_kernel(FlashArgs a) {
     }
 }
 
+// The rows that one P.V wave of the PV64 layout holds at the end of its pass: O[2 cb + t] is
+// column block cb (32 of the wave's columns 128cq .. +127) of row tile t, its lane holding 4
+// columns 8q + 4(l/32) .. of row l%32.  They go out through the wave's part of the ring, which
+// is free by then, in whole 512-byte (normalised 16-bit: 256-byte) pieces of a row: straight
+// from the registers they were stores of 16 bytes a row, 32 rows an instruction.
+//   fp32: chunk c of row r at c ^ (r & 15) of its 512 bytes; 16-bit: chunk c at c ^ (r & 15) of
+//   256 bytes, the two halves of a chunk swapped in rows with bit 4 set: the writes of 32 rows
+//   and the reads touch all banks evenly.
+constexpr uint32_t kPvOutBytes = 64 * 512;
+template <typename TL>
+__device__ __forceinline__ void pv_store_rows(const FlashArgs& a, const FlashWork& work,
+                                              uint8_t* mine, const v16f (&O)[8], const float* xl,
+                                              const float* xref, int r0, int rows_b, int cq,
+                                              int lane, float of) {
+    const int l32 = lane & 31, hw = lane >> 5;
+    const bool norm = a.ctx16 && (work.direct || (!a.wl && a.n_split == 1));
+    const int64_t slot0 = (work.direct ? (int64_t)work.b : work.slot) * rows_b + r0;
+    const int rows = rows_b - r0;   // of the tile, if below 64
+    #pragma unroll
+    for (int t = 0; t < 2; ++t) {
+        const int row = 32 * t + l32;
+        const float lsum = xl[t * 64 + l32] + xl[t * 64 + 32 + l32];
+        if (norm) {
+            const float r = lsum == 0.f ? 0.f : 1.f / lsum;
+            #pragma unroll
+            for (int cb = 0; cb < 4; ++cb)
+                #pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    const v4f v = v4f{O[2 * cb + t][4 * q], O[2 * cb + t][4 * q + 1],
+                                      O[2 * cb + t][4 * q + 2], O[2 * cb + t][4 * q + 3]} * of;
+                    const v4f w = v * r;
+                    *reinterpret_cast<v2u*>(mine + row * 256 + 16 * ((4 * cb + q) ^ (row & 15)) +
+                                            8 * (hw ^ ((row >> 4) & 1))) =
+                        v2u{Half<TL>::pack2(w[0], w[1]), Half<TL>::pack2(w[2], w[3])};
+                }
+        } else {
+            if (cq == 0 && hw == 0 && row < rows) {
+                if (!work.direct) a.m[slot0 + row] = xref[t * 64 + l32];
+                (work.direct ? a.l_direct : a.l)[slot0 + row] = lsum;
+            }
+            #pragma unroll
+            for (int cb = 0; cb < 4; ++cb)
+                #pragma unroll
+                for (int q = 0; q < 4; ++q)
+                    *reinterpret_cast<v4f*>(mine + row * 512 + 16 * ((8 * cb + 2 * q + hw) ^ (row & 15))) =
+                        v4f{O[2 * cb + t][4 * q], O[2 * cb + t][4 * q + 1], O[2 * cb + t][4 * q + 2],
+                            O[2 * cb + t][4 * q + 3]} * of;
+        }
+    }
+    __builtin_amdgcn_wave_barrier();
+    if (norm) {
+        uint16_t* const dst = static_cast<uint16_t*>(a.ctx16) + slot0 * kFR + 128 * cq + 8 * (lane & 15);
+        #pragma unroll
+        for (int i = 0; i < 16; ++i) {
+            const int row = 4 * i + (lane >> 4);
+            const v4u v = *reinterpret_cast<const v4u*>(mine + row * 256 + 16 * ((lane & 15) ^ (row & 15)));
+            if (row < rows)
+                *reinterpret_cast<v4u*>(dst + (int64_t)row * kFR) = (i >> 2) & 1 ? v4u{v[2], v[3], v[0], v[1]} : v;
+        }
+    } else {
+        float* const dst = (work.direct ? a.o_direct : a.o) + slot0 * kFR + 128 * cq + 4 * l32;
+        #pragma unroll
+        for (int i = 0; i < 32; ++i) {
+            const int row = 2 * i + hw;
+            const v4f v = *reinterpret_cast<const v4f*>(mine + row * 512 + 16 * (l32 ^ (row & 15)));
+            if (row < rows) *reinterpret_cast<v4f*>(dst + (int64_t)row * kFR) = v;
+        }
+    }
+}
+
 // ------------------------------------------------------------------ 16-bit: specialised waves
 // The same 64-row tile, 32-key blocks, staging and LDS ring as flash16_kernel, on eight
 // waves whose work is split by kind instead of by key half (two waves per SIMD, so one
@@ -787,21 +857,6 @@ __global__ void __launch_bounds__(kXThreads, 1) flash16x_kernel(FlashArgs a) {
             lim1 = min(lim1, skb - a.Sq + min(rowS1, rows_b - 1) / a.H);
         }
         const int lim_wave = __builtin_amdgcn_readfirstlane(lim0);
-        const __amdgpu_buffer_rsrc_t rq = make_rsrc(a.qa + (int64_t)b * rows_b * kFR);
-        const __amdgpu_buffer_rsrc_t rr = make_rsrc(a.qr + (int64_t)b * rows_b * kFD);
-        v4u qf[2][kQSteps];
-        #pragma unroll
-        for (int t = 0; t < 2; ++t) {
-            const int row = t ? rowS1 : rowS0;
-            const uint32_t qmask = oob_mask(row, rows_b);
-            #pragma unroll
-            for (int s = 0; s < kQSteps; ++s)
-                qf[t][s] = s < kRSteps
-                               ? load16(rq, ((uint32_t)row * kLatBytes + 256u * g + 16u * s) | qmask)
-                               : load16(rr, ((uint32_t)row * kPeBytes + 64u * (s - kRSteps) + 16u * g) | qmask);
-        }
-        wait_vm<0>();   // Q in registers
-
         const int kk = 16 * kh + l16;
         uint32_t kb0 = kk * kLatBytes + 256u * g + 16u * sw16(l16);
         uint32_t pb0 = kPeBase + kk * kPeBytes + 16u * (g ^ ((kk >> 1) & 7));
@@ -809,6 +864,33 @@ __global__ void __launch_bounds__(kXThreads, 1) flash16x_kernel(FlashArgs a) {
             const uint32_t off = s < kRSteps ? (kbs ^ (16u * s)) : (pbs ^ (64u * (s - kRSteps)));
             return *reinterpret_cast<const v4u*>(smem + off);
         };
+        v4u qf[2][kQSteps];
+        if constexpr (FP8) {
+            const __amdgpu_buffer_rsrc_t rq = make_rsrc(a.qa + (int64_t)b * rows_b * kFR);
+            const __amdgpu_buffer_rsrc_t rr = make_rsrc(a.qr + (int64_t)b * rows_b * kFD);
+            #pragma unroll
+            for (int t = 0; t < 2; ++t) {
+                const int row = t ? rowS1 : rowS0;
+                const uint32_t qmask = oob_mask(row, rows_b);
+                #pragma unroll
+                for (int s = 0; s < kQSteps; ++s)
+                    qf[t][s] = s < kRSteps
+                                   ? load16(rq, ((uint32_t)row * kLatBytes + 256u * g + 16u * s) | qmask)
+                                   : load16(rr, ((uint32_t)row * kPeBytes + 64u * (s - kRSteps) + 16u * g) | qmask);
+            }
+            wait_vm<0>();   // Q in registers
+        } else if (nb > 0) {
+            // Q: rows 32rt .. +31 of the tile lie in ring stage 2 + rt like a block's keys
+            lds_barrier();   // Q: the P.V waves' query loads have landed
+            #pragma unroll
+            for (int t = 0; t < 2; ++t) {
+                const int qk = 16 * t + l16;
+                const uint32_t qb = lat_base(qk * kLatBytes + 256u * g + 16u * sw16(l16), 2 + rt);
+                const uint32_t qp = kPeBase + (2 + rt) * k2PeStage + qk * kPeBytes + 16u * (g ^ ((qk >> 1) & 7));
+                #pragma unroll
+                for (int s = 0; s < kQSteps; ++s) qf[t][s] = k_read(qb, qp, s);
+            }
+        }
         // P^T writes: rows 16h + l16 of the tile, keys 16kh + 4g .. +3 (8 bytes)
         const uint32_t pw0 = kPBase + rt * 32 * kXPPitch + l16 * kXPPitch + 2u * (16 * kh + 4 * g);
 
@@ -1005,6 +1087,34 @@ __global__ void __launch_bounds__(kXThreads, 1) flash16x_kernel(FlashArgs a) {
     auto f8_write = [&](int j, int q, v4u raw) __attribute__((always_inline)) {
         f8.write(smem, j % NS, q, raw, lane);
     };
+    if constexpr (!FP8) {
+        // The tile's queries, in rows of 1 KB like the keys, into ring stages 2 and 3 (free
+        // until block 2 is issued, after barrier A_0): wave w loads rows 16w .. 16w+15.  The
+        // score waves read their fragments from there in the K fragments' pattern.  Loaded
+        // from global memory straight into those fragments, each 16-byte piece of a row came
+        // in a load of its own (64 lines an instruction, 144 instructions a workgroup).  With
+        // the rows' way out (pv_store_rows) one block at B = 128 takes 13.0 us, was 16.0; the
+        // causal B = 1, Sq = Sk = 4096 attention 2,320 -> 2,232 us, an fp16 layer of 64 x 4
+        // queries 172.0 -> 166.6 us.
+        if (nb > 0) {
+            const uint32_t rows_q = (uint32_t)min(kFRows, rows_b - r0), row0 = 16 * wv;
+            const v4i rq = rsrc_span(reinterpret_cast<uint64_t>(a.qa + ((int64_t)b * rows_b + r0) * kFR),
+                                     0, rows_q * kLatBytes);
+            const v4i rr = rsrc_span(reinterpret_cast<uint64_t>(a.qr + ((int64_t)b * rows_b + r0) * kFD),
+                                     0, rows_q * kPeBytes);
+            const uint32_t slot0 = 16 * (wv & 1), st = 2 + (wv >> 1);
+            const uint32_t ql = __builtin_amdgcn_readfirstlane(lds0 + st * k2LatStage + slot0 * kLatBytes);
+            const uint32_t qp = __builtin_amdgcn_readfirstlane(lds0 + kPeBase + st * k2PeStage + slot0 * kPeBytes);
+            #pragma unroll
+            for (int q = 0; q < 16; ++q)
+                dma16(rq, ql + q * kLatBytes, lane16 ^ (16u * sw16(q)), (row0 + q) * kLatBytes);
+            #pragma unroll
+            for (int q = 0; q < 2; ++q)
+                dma16(rr, qp + q * 1024,
+                      (uint32_t)(lane >> 3) * kPeBytes + 16u * ((lane & 7) ^ ((4 * q + (lane >> 4)) & 7)),
+                      (row0 + 8 * q) * kPeBytes);
+        }
+    }
     v16f O[8];
     for (int pass = 1;; ++pass) {
         #pragma unroll
@@ -1015,6 +1125,12 @@ __global__ void __launch_bounds__(kXThreads, 1) flash16x_kernel(FlashArgs a) {
             const Loads d = loads_of(j);
             #pragma unroll
             for (int q = 0; q < kLoads; ++q) issue_one(d, q);
+        }
+        if constexpr (!FP8) {
+            if (pass == 1) {
+                wait_vm<2 * kLoads>();     // the queries have landed
+                lds_barrier();             // Q
+            }
         }
         wait_vm<kLoads>();                 // block 0 has landed; block 1 may be in flight
         if constexpr (FP8) {               // block 0 into the bf16 ring
@@ -1112,43 +1228,7 @@ __global__ void __launch_bounds__(kXThreads, 1) flash16x_kernel(FlashArgs a) {
     // an fp8 cache's values are its codes times kv_scale: ctx takes the factor here
     const float of = FP8 ? a.o_scale : 1.f;
     if constexpr (PV64) {
-        // both row tiles, columns 128cq .. +127: O[2 cb + t] is column block cb of row tile t
-        #pragma unroll
-        for (int t = 0; t < 2; ++t) {
-            const int row = r0 + 32 * t + l32;
-            if (row >= rows_b) continue;
-            const float* xlr = xl + t * 64;
-            const float lsum = xlr[l32] + xlr[32 + l32];
-            const float M = xref[t * 64 + l32];
-            const int64_t slot = (work.direct ? (int64_t)b : work.slot) * rows_b + row;
-            if (a.ctx16 && (work.direct || (!a.wl && a.n_split == 1))) {
-                const float r = lsum == 0.f ? 0.f : 1.f / lsum;
-                uint16_t* crow = static_cast<uint16_t*>(a.ctx16) + slot * kFR + 128 * cq + 4 * hw;
-                #pragma unroll
-                for (int cb = 0; cb < 4; ++cb)
-                    #pragma unroll
-                    for (int q = 0; q < 4; ++q) {
-                        const v4f v = v4f{O[2 * cb + t][4 * q], O[2 * cb + t][4 * q + 1],
-                                          O[2 * cb + t][4 * q + 2], O[2 * cb + t][4 * q + 3]} * of;
-                        const v4f w = v * r;
-                        *reinterpret_cast<v2u*>(crow + 32 * cb + 8 * q) =
-                            v2u{Half<TL>::pack2(w[0], w[1]), Half<TL>::pack2(w[2], w[3])};
-                    }
-                continue;
-            }
-            if (cq == 0 && hw == 0) {
-                if (!work.direct) a.m[slot] = M;
-                (work.direct ? a.l_direct : a.l)[slot] = lsum;
-            }
-            float* orow = (work.direct ? a.o_direct : a.o) + slot * kFR + 128 * cq + 4 * hw;
-            #pragma unroll
-            for (int cb = 0; cb < 4; ++cb)
-                #pragma unroll
-                for (int q = 0; q < 4; ++q)
-                    *reinterpret_cast<v4f*>(orow + 32 * cb + 8 * q) =
-                        v4f{O[2 * cb + t][4 * q], O[2 * cb + t][4 * q + 1],
-                            O[2 * cb + t][4 * q + 2], O[2 * cb + t][4 * q + 3]} * of;
-        }
+        pv_store_rows<TL>(a, work, smem + cq * kPvOutBytes, O, xl, xref, r0, rows_b, cq, lane, of);
     } else if (rowO < rows_b) {
         const float* xlr = xl + rt * 64;
         const float lsum = xlr[l32] + xlr[32 + l32];
@@ -1214,6 +1294,10 @@ __global__ void __launch_bounds__(kXThreads, 1) flash16x8_kernel(FlashArgs a) {
     typedef bf16_t TL;
     constexpr float kHeadroom = k2Headroom;
     constexpr int kPBase = k8NS * k8Stage;                      // 144 KB: two P^T stages
+    // the queries at the start: 64 rows of 1 KB (chunk c of row r at c ^ (r & 15)), then 64 rope
+    // rows of 128 bytes (chunk c at c ^ ((r >> 1) & 7)), in the last four stages
+    constexpr int kQBase = 4 * k8Stage;
+    static_assert(kFRows * (kLatBytes + kPeBytes) == 4 * k8Stage, "the queries fill four stages");
     constexpr int kXBase = kPBase + 2 * kXPStage;               // references, sums, flags
     __shared__ __attribute__((aligned(1024))) uint8_t smem[kXBase + 2 * 128 * 4 + 64];
     float* xref = reinterpret_cast<float*>(smem + kXBase);      // [rt][kh][32 rows]
@@ -1246,21 +1330,22 @@ __global__ void __launch_bounds__(kXThreads, 1) flash16x8_kernel(FlashArgs a) {
             lim1 = min(lim1, skb - a.Sq + min(rowS1, rows_b - 1) / a.H);
         }
         const int lim_wave = __builtin_amdgcn_readfirstlane(lim0);
-        const __amdgpu_buffer_rsrc_t rq = make_rsrc(a.qa + (int64_t)b * rows_b * kFR);
-        const __amdgpu_buffer_rsrc_t rr = make_rsrc(a.qr + (int64_t)b * rows_b * kFD);
-        // Q^T fragments: step s of lane group g is depth 32s + 8g .. +7 (bf16: 16 bytes)
+        // Q^T fragments: step s of lane group g is depth 32s + 8g .. +7 (bf16: 16 bytes), chunk
+        // 4s + g of the row (rope: 4 (s - 16) + g), from the ring's last four stages
         v4u qf[2][kQSteps];
-        #pragma unroll
-        for (int t = 0; t < 2; ++t) {
-            const int row = t ? rowS1 : rowS0;
-            const uint32_t qmask = oob_mask(row, rows_b);
+        if (nb > 0) {
+            lds_barrier();   // Q: the P.V waves' query loads have landed
             #pragma unroll
-            for (int s = 0; s < kQSteps; ++s)
-                qf[t][s] = s < kRSteps
-                               ? load16(rq, ((uint32_t)row * kLatBytes + 64u * s + 16u * g) | qmask)
-                               : load16(rr, ((uint32_t)row * kPeBytes + 64u * (s - kRSteps) + 16u * g) | qmask);
+            for (int t = 0; t < 2; ++t) {
+                const int row = 32 * rt + 16 * t + l16;
+                const uint32_t ql = kQBase + row * kLatBytes + 16u * (g ^ (row & 15));
+                const uint32_t qp = kQBase + kFRows * kLatBytes + row * kPeBytes + 16u * (g ^ ((row >> 1) & 7));
+                #pragma unroll
+                for (int s = 0; s < kQSteps; ++s)
+                    qf[t][s] = *reinterpret_cast<const v4u*>(
+                        smem + (s < kRSteps ? ql ^ (64u * s) : qp ^ (64u * (s - kRSteps))));
+            }
         }
-        wait_vm<0>();   // Q in registers
 
         // K step s: bytes 32s + 8g of key kk's latent row, i.e. chunk 2s + g/2 at position
         // (2s + g/2) ^ x, x = swz(kk & 15): 32 (s ^ x/2) + 16 (g/2 ^ x%2) + 8 (g%2); the rope
@@ -1462,16 +1547,40 @@ __global__ void __launch_bounds__(kXThreads, 1) flash16x8_kernel(FlashArgs a) {
         if (pe_loader) wait_vm<5 * n>();
         else wait_vm<4 * n>();
     };
+    // The tile's queries into the last four stages, free until block 4 is issued after barrier
+    // A_0: wave w loads rows 16w .. 16w+15.
+    if (nb > 0) {
+        const uint32_t rows_q = (uint32_t)min(kFRows, rows_b - r0), row0 = 16 * wv;
+        const v4i rq = rsrc_span(reinterpret_cast<uint64_t>(a.qa + ((int64_t)b * rows_b + r0) * kFR), 0,
+                                 rows_q * kLatBytes);
+        const v4i rr = rsrc_span(reinterpret_cast<uint64_t>(a.qr + ((int64_t)b * rows_b + r0) * kFD), 0,
+                                 rows_q * kPeBytes);
+        const uint32_t ql = __builtin_amdgcn_readfirstlane(lds0 + kQBase + row0 * kLatBytes);
+        const uint32_t qp = __builtin_amdgcn_readfirstlane(lds0 + kQBase + kFRows * kLatBytes + row0 * kPeBytes);
+        #pragma unroll
+        for (int q = 0; q < 16; ++q)
+            dma16(rq, ql + q * kLatBytes, 16u * (lane ^ q), (row0 + q) * kLatBytes);
+        #pragma unroll
+        for (int q = 0; q < 2; ++q)
+            dma16(rr, qp + q * 1024,
+                  (uint32_t)(lane >> 3) * kPeBytes + 16u * ((lane & 7) ^ ((4 * q + (lane >> 4)) & 7)),
+                  (row0 + 8 * q) * kPeBytes);
+    }
     v16f O[8];
     for (int pass = 1;; ++pass) {
         #pragma unroll
         for (int i = 0; i < 8; ++i) O[i] = v16f{};
         if (nb == 0) break;
         #pragma unroll
-        for (int j = 0; j < k8Ahead; ++j) issue_block(loads_of(j));
-        wait_blocks(std::integral_constant<int, k8Ahead - 1>{});   // block 0 has landed
+        for (int j = 0; j < 4; ++j) issue_block(loads_of(j));
+        if (pass == 1) {
+            wait_blocks(std::integral_constant<int, 4>{});   // the queries have landed
+            lds_barrier();                 // Q
+        }
+        wait_blocks(std::integral_constant<int, 3>{});       // block 0 has landed
         lds_barrier();                     // A_0
-        issue_block(loads_of(k8Ahead));    // its stage is free from the pass's start
+        #pragma unroll
+        for (int j = 4; j <= k8Ahead; ++j) issue_block(loads_of(j));   // their stages are free now
         lds_barrier();                     // X
         #pragma unroll 1
         for (int j = 1; j <= nb; ++j) {
@@ -1518,44 +1627,8 @@ __global__ void __launch_bounds__(kXThreads, 1) flash16x8_kernel(FlashArgs a) {
         if (!again) break;
     }
     lds_barrier();       // F
-    // both row tiles, columns 128cq .. +127: O[2 cb + t] is column block cb of row tile t; an
-    // fp8 cache's values are its codes times kv_scale, so ctx takes the factor here
-    #pragma unroll
-    for (int t = 0; t < 2; ++t) {
-        const int row = r0 + 32 * t + l32;
-        if (row >= rows_b) continue;
-        const float* xlr = xl + t * 64;
-        const float lsum = xlr[l32] + xlr[32 + l32];
-        const float M = xref[t * 64 + l32];
-        const int64_t slot = (work.direct ? (int64_t)b : work.slot) * rows_b + row;
-        if (a.ctx16 && (work.direct || (!a.wl && a.n_split == 1))) {
-            const float r = lsum == 0.f ? 0.f : 1.f / lsum;
-            uint16_t* crow = static_cast<uint16_t*>(a.ctx16) + slot * kFR + 128 * cq + 4 * hw;
-            #pragma unroll
-            for (int cb = 0; cb < 4; ++cb)
-                #pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    const v4f v = v4f{O[2 * cb + t][4 * q], O[2 * cb + t][4 * q + 1],
-                                      O[2 * cb + t][4 * q + 2], O[2 * cb + t][4 * q + 3]} * a.o_scale;
-                    const v4f w = v * r;
-                    *reinterpret_cast<v2u*>(crow + 32 * cb + 8 * q) =
-                        v2u{Half<bf16_t>::pack2(w[0], w[1]), Half<bf16_t>::pack2(w[2], w[3])};
-                }
-            continue;
-        }
-        if (cq == 0 && hw == 0) {
-            if (!work.direct) a.m[slot] = M;
-            (work.direct ? a.l_direct : a.l)[slot] = lsum;
-        }
-        float* orow = (work.direct ? a.o_direct : a.o) + slot * kFR + 128 * cq + 4 * hw;
-        #pragma unroll
-        for (int cb = 0; cb < 4; ++cb)
-            #pragma unroll
-            for (int q = 0; q < 4; ++q)
-                *reinterpret_cast<v4f*>(orow + 32 * cb + 8 * q) =
-                    v4f{O[2 * cb + t][4 * q], O[2 * cb + t][4 * q + 1], O[2 * cb + t][4 * q + 2],
-                        O[2 * cb + t][4 * q + 3]} * a.o_scale;
-    }
+    // an fp8 cache's values are its codes times kv_scale: ctx takes the factor here
+    pv_store_rows<TL>(a, work, smem + cq * kPvOutBytes, O, xl, xref, r0, rows_b, cq, lane, a.o_scale);
 }
 
 // ------------------------------------------------------------------ fp32 variant
