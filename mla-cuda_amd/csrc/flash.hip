@@ -2630,7 +2630,7 @@ __global__ void __launch_bounds__(kWlThreads) flash_worklist_kernel(const int* _
     // decode step's critical path
     static_assert(kWlThreads == 256 && kWlBuckets == 256, "one bucket per thread, four waves");
     __shared__ long long w_tot[4];
-    __shared__ int w_min[4], w_max[4], w_cnt[4], w_full[4], w_rem[4];
+    __shared__ int w_min[4], w_max[4], w_cnt[4], w_full[4], w_rem[4], w_try[4][kWlTries], w_small[4][kWlTries];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int b0 = wl_thread_first(tid, B), b1 = wl_thread_first(tid + 1, B);
     // a thread's lengths stay in registers (up to 8 batches per thread, B <= 2048); past
@@ -2667,7 +2667,36 @@ __global__ void __launch_bounds__(kWlThreads) flash_worklist_kernel(const int* _
     tot = ((w_tot[0] + w_tot[1]) + w_tot[2]) + w_tot[3];
     mn = min(min(w_min[0], w_min[1]), min(w_min[2], w_min[3]));
     mx = max(max(w_max[0], w_max[1]), max(w_max[2], w_max[3]));
-    int chunk = wl_initial_chunk(tot, mn, mx, B, Sk, row_tiles, block_keys);
+    int chunk;
+    if (mn == mx) {
+        chunk = dense_keys_per_split(wl_max(1, mx), B * row_tiles, block_keys);
+    } else {
+        // every candidate's piece count in one pass; all threads then pick the same one
+        const int base = wl_base_blocks(tot, row_tiles, block_keys);
+        #pragma unroll
+        for (int k = 0; k < kWlTries; ++k) {
+            const int c = wl_try(base, k, Sk, block_keys);
+            int n = 0, small = 0;
+            for (int b = b0; b < b1; ++b) {
+                const int L = len_of(b);
+                n += wl_chunk_count(L, c);
+                small += wl_small(L, c, block_keys);
+            }
+            for (int d = 32; d > 0; d >>= 1) {
+                n += __shfl_xor(n, d);
+                small += __shfl_xor(small, d);
+            }
+            if (lane == 0) { w_try[wave][k] = n; w_small[wave][k] = small; }
+        }
+        __syncthreads();
+        int k = 0;
+        for (; k < kWlTries - 1; ++k) {
+            long long n = 0, small = 0;
+            for (int w = 0; w < 4; ++w) { n += w_try[w][k]; small += w_small[w][k]; }
+            if (wl_packs(n, small, tot, wl_try(base, k, Sk, block_keys), row_tiles, block_keys)) break;
+        }
+        chunk = wl_try(base, k, Sk, block_keys);
+    }
     int cnt, full;
     for (;;) {
         cnt = 0; full = 0;

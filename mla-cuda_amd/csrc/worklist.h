@@ -28,17 +28,8 @@
 namespace mla {
 
 constexpr int kWlHead = 2;
-// A ragged list spreads the total key count over kWlPerCu workgroups per CU (fp32) or
-// kWlPerCu16 (bf16, fp16 and the fp8 cache).  At B=128 with lengths uniform in [1, 4989],
-// fp32: 1 per CU took 1185 us, 2: 950, 3: 901, 4: 870-905, 6: 926, 8: 907 (more pieces
-// shorten the tail; each piece costs its Q load and partials).  16-bit: 1 per CU took
-// 150.5 us, 2: 165.7, 3: 185.4, 4: 202.4 (fp8 cache 186.3 / 208.1 / 229.9 / 254.2; one
-// sequence of 4989 keys per seven of 300: bf16 95.7 us at 1 against 153.9 at 4): a 16-bit
-// key block is ~5x shorter than an fp32 one, so a piece's fixed cost weighs ~5x more.
-// The list is sized for the larger kWlPerCu.
+// Sizes of a ragged list: its items and partial slots hold kWlPerCu pieces per CU.
 constexpr int kWlPerCu = 4;
-constexpr int kWlPerCu16 = 1;
-static_assert(kWlPerCu16 <= kWlPerCu, "the list is sized for kWlPerCu pieces per CU");
 constexpr int kWlBuckets = 256;     // length buckets of the last-chunk counting sort
 constexpr int kWlThreads = 256;     // threads of the device builder
 
@@ -47,8 +38,8 @@ MLA_HD int wl_max(int a, int b) { return a > b ? a : b; }
 
 MLA_HD int wl_ints(int B, int max_items) { return kWlHead + 2 * B + 2 * max_items; }
 
-// Items of a balanced list: at most kWlPerCu * CUs / row_tiles + B (either chunk rule of
-// wl_initial_chunk), rounded up to a whole number per XCD.
+// Items of a balanced list: kWlPerCu * CUs / row_tiles + B (no chunk rule gives more), rounded
+// up to a whole number per XCD.
 MLA_HD int wl_max_items(int B, int row_tiles) {
     return (kWlPerCu * kNumCUs / row_tiles + B + 1 + kNumXCDs - 1) / kNumXCDs * kNumXCDs;
 }
@@ -114,22 +105,52 @@ MLA_HD int wl_bucket(int L, int chunk) {
     return (int)(((long long)(chunk - 1 - r) * kWlBuckets) / chunk);
 }
 
-// Chunk before the fit check, from the batch's total, minimum and maximum key counts:
-//   every sequence the same length L -> the dense plan's keys per split for L, so the list
-//     reproduces the dense launch exactly (same key ranges, same merge order);
-//   otherwise -> the total key count spread over kWlPerCu (fp32, 16-key blocks) or
-//     kWlPerCu16 (16-bit, 32-key blocks) workgroups per CU (a multiple of the key block,
-//     so a wave's keys never straddle a page; at least 4 blocks; at most the key span
-//     rounded up to a block).
-MLA_HD int wl_initial_chunk(long long tot, int mn, int mx, int B, int Sk, int row_tiles,
-                            int block_keys) {
-    if (mn == mx) return dense_keys_per_split(wl_max(1, mx), B * row_tiles, block_keys);
-    const long long wgs = (long long)(block_keys == 16 ? kWlPerCu : kWlPerCu16) * kNumCUs;
-    const long long want = (tot * row_tiles + wgs - 1) / wgs;
-    const long long cap = (long long)(Sk + block_keys - 1) / block_keys * block_keys;
-    long long chunk = (want + block_keys - 1) / block_keys * block_keys;
-    chunk = chunk < cap ? chunk : cap;
-    return wl_max((int)chunk, 4 * block_keys);
+// Chunk before the fit check.  Every sequence the same length L: the dense plan's keys per
+// split for L, so the list reproduces the dense launch exactly (same key ranges, same merge
+// order).  Otherwise it is chosen for the time the last workgroup ends.  A piece costs its key
+// blocks and a fixed part (queries, first loads, the rows' way out, its share of the merge):
+// about 11 blocks of 32 keys in 16-bit, 4 of 16 keys in fp32.  The pieces are dispatched longest
+// first, so the grid ends about when one full chunk does if every piece has a CU, or if the
+// pieces pack beside the full ones:
+//   (pieces * fixed + blocks) * row_tiles <= 96% of CUs * (fixed + chunk), and
+//   as many short pieces as are left over fit twice into one chunk's time
+//   (length <= (chunk - fixed) / 2).
+// The first of kWlTries chunks that meets this is taken, from an equal share of the blocks per
+// CU (wl_base_blocks) up in steps of 1/16 of it.  Where that share is longer than any sequence,
+// 16-bit sequences stay whole and fp32 ones are cut at a quarter of it.
+// Read from caches too large to keep, against the former rules (the share itself in 16-bit, a
+// quarter of it in fp32), attention with 3d, lengths uniform up to the figure: bf16 B = 61, 4,989
+// 91.5 -> 87.3 us, B = 16, 8,192 66.4 -> 59.6, B = 32, 8,192 81.2 -> 71.3; fp8 B = 32, 8,192
+// 82.6 -> 72.4; fp32 B = 128, 4,989 772 -> 744, B = 32 286 -> 226; one sequence of 4,989 keys
+// per seven of 300, B = 64: fp32 261 -> 210.  In a simulation of the dispatch over 132 length
+// distributions (B = 5..300) the grid ends 12% sooner in 16-bit, 18% in fp32, never over 5% later.
+constexpr int kWlTries = 8;
+MLA_HD int wl_fixed_blocks(int block_keys) { return block_keys == 16 ? 4 : 11; }
+MLA_HD int wl_base_blocks(long long tot, int row_tiles, int block_keys) {
+    const long long per = (tot * row_tiles + kNumCUs - 1) / kNumCUs;
+    const long long blocks = (per + block_keys - 1) / block_keys;
+    return blocks < 4 ? 4 : blocks > 0x3fffffff ? 0x3fffffff : (int)blocks;
+}
+// Keys of candidate k: at most the key span rounded up to a block, at least 4 blocks.
+MLA_HD int wl_try(int base_blocks, int k, int Sk, int block_keys) {
+    const int cap = wl_max((Sk + block_keys - 1) / block_keys, 4);
+    if (base_blocks >= cap)
+        return (block_keys == 16 ? wl_max(4, wl_min(cap, (base_blocks + 3) / 4)) : cap) * block_keys;
+    const long long blocks = ((long long)base_blocks * (16 + k) + 15) / 16;
+    return (int)(blocks < cap ? blocks : cap) * block_keys;
+}
+// Whether a sequence's last chunk is short enough to share a CU with another piece.
+MLA_HD int wl_small(int L, int chunk, int block_keys) {
+    return wl_has_short(L, chunk) && 2 * (L % chunk) <= chunk - wl_fixed_blocks(block_keys) * block_keys;
+}
+// Whether `pieces` chunks, `small` of them by wl_small, `tot` keys in all, pack (see above).
+MLA_HD bool wl_packs(long long pieces, long long small, long long tot, int chunk, int row_tiles,
+                     int block_keys) {
+    const long long left = pieces * row_tiles - kNumCUs;
+    if (left <= 0) return true;
+    const long long f = wl_fixed_blocks(block_keys);
+    return small * row_tiles >= left &&
+           100 * (pieces * f + tot / block_keys) * row_tiles <= 96LL * kNumCUs * (f + chunk / block_keys);
 }
 
 // The list must fit max_items (the partial slots and the grid are sized for it).  A chunk
@@ -193,7 +214,17 @@ inline int wl_build_serial(const int* seq_lens, int B, int Sk, int row_tiles, in
         mn = wl_min(mn, L);
         mx = wl_max(mx, L);
     }
-    int chunk = wl_initial_chunk(tot, mn, mx, B, Sk, row_tiles, block_keys);
+    int chunk = mn == mx ? dense_keys_per_split(wl_max(1, mx), B * row_tiles, block_keys) : 0;
+    for (int k = 0; mn != mx && k < kWlTries; ++k) {
+        chunk = wl_try(wl_base_blocks(tot, row_tiles, block_keys), k, Sk, block_keys);
+        long long pieces = 0, small = 0;
+        for (int b = 0; b < B; ++b) {
+            const int L = wl_len(seq_lens[b], Sk);
+            pieces += wl_chunk_count(L, chunk);
+            small += wl_small(L, chunk, block_keys);
+        }
+        if (wl_packs(pieces, small, tot, chunk, row_tiles, block_keys)) break;
+    }
     long long total;
     int n_full;
     for (;;) {

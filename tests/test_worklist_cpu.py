@@ -147,3 +147,26 @@ def test_spread_tiles_cover_once_and_balance(units, row_tiles):
     for p, t in enumerate(got[:n]):
         work[p % 8] += t % row_tiles + 1
     assert work.max() <= work.mean() + row_tiles * (units / 8 + 1) / 8 + row_tiles
+
+
+@pytest.mark.parametrize("block_keys", [16, 32])
+@pytest.mark.parametrize("B,lo,hi", [(16, 1, 8192), (61, 1, 4989), (64, 300, 4989), (200, 1, 2000)])
+def test_ragged_chunk_packs_or_is_the_last_candidate(block_keys, B, lo, hi):
+    """A ragged batch's chunk lies between an equal share of the key blocks per CU and 23/16
+    of it, and below the last candidate its pieces meet the packing condition, restated here."""
+    rng = np.random.default_rng(B + hi)
+    lens = rng.integers(lo, hi + 1, B)
+    if lo == 300:
+        lens = np.where(np.arange(B) % 8 == 0, hi, lo)
+    Sk, rt, fixed = -(-hi // 64) * 64, 2, 4 if block_keys == 16 else 11
+    chunk = int(W.build_serial(lens, Sk, rt, block_keys)[1])
+    share = max(4, -(-(-(-int(lens.sum()) * rt // 256)) // block_keys))
+    cap = -(-Sk // block_keys)
+    assert share < cap and share * block_keys <= chunk <= min(cap, -(-share * 23 // 16)) * block_keys
+    if chunk // block_keys < min(cap, -(-share * 23 // 16)):
+        n = sum(-(-int(l) // chunk) for l in lens)
+        short = [int(l) % chunk for l in lens if int(l) % chunk]
+        small = sum(2 * s <= chunk - fixed * block_keys for s in short)
+        assert n * rt <= 256 or (small * rt >= n * rt - 256 and
+                                 (n * fixed + int(lens.sum()) // block_keys) * rt
+                                 <= 0.96 * 256 * (fixed + chunk // block_keys))
