@@ -829,19 +829,20 @@ bool wgemm_rule(const GemmProblem& p, GemmPlan* out) {
     return best < 1e300;
 }
 
-// Large tiles, M > 128.  A workgroup's time is its 32-deep slices at the tile's slice time --
-// of a lightly loaded chip, and what a full one adds as its clock drops -- plus ~5.6 us of
-// launch, first loads and stores; rounds of 256 workgroups (128 x 128: two per CU, where one's
-// stores pass under the other's MFMAs: 4 us).  Fitted to 500 measured (shape, plan) pairs of
-// the four weight products at M = 160..4096 (9% rms; the plan it picks is within 10% of the
-// best measured one everywhere, and the best at most).  3d (N = 128, K = 512) takes 128 x 128
-// (M = 4096: 188 against 214 us on 256 x 128), 2c (K = 128) 256 x 256 (M = 2048: 111-116
-// against 157 on 256 x 128 and 129 on 128 x 128).
+// Large tiles, M > 128.  A tile's time is its 32-deep slices at the tile's slice time -- of a
+// lightly loaded chip, and what a full one adds as its clock drops; a workgroup (256 at a time,
+// 128 x 128: two per CU) adds ~5.6 us of launch, first loads and last stores, and ~3 us of
+// results for each further tile.  Fitted to 500 measured (shape, plan) pairs of the four weight
+// products at M = 160..4096 (9% rms; the plan it picks is within 10% of the best measured one
+// everywhere, and the best at most).  The grouped products follow it too: 3d (N = 128, K = 512)
+// takes 256 x 128 at M = 4096 (155 against 173 us on 128 x 128) and 128 x 128 at M = 256 (13.5
+// against 18), 2c (K = 128) 256 x 256 (M = 2048: 93-102 against 114 and 126).
 bool bgemm_rule(const GemmProblem& p, GemmPlan* out) {
     if (p.M <= kStreamRows) return false;
-    struct Tile { int bm, bn, per_cu; double slice, load, fixed; };   // us
-    constexpr Tile kBTiles[] = {{256, 256, 1, 0.56, 0.25, 5.6}, {256, 128, 1, 0.40, 0.14, 5.6},
-                                {128, 128, 2, 0.19, 0.21, 4.0}};
+    struct Tile { int bm, bn, per_cu; double slice, load; };   // us
+    constexpr Tile kBTiles[] = {{256, 256, 1, 0.56, 0.25}, {256, 128, 1, 0.40, 0.14},
+                                {128, 128, 2, 0.19, 0.21}};
+    constexpr double kFirst = 5.6, kNext = 3.0;
     const int kslices = cdiv(p.K, 64), most = max_split(p, kslices);
     double best = 1e300;
     for (const Tile& b : kBTiles)
@@ -851,12 +852,12 @@ bool bgemm_rule(const GemmProblem& p, GemmPlan* out) {
             const double nsl = 2.0 * per;
             const int64_t wgs = (int64_t)cdiv(p.M, b.bm) * cdiv(p.N, b.bn) * p.G * split;
             const int64_t cap = (int64_t)kNumCUs * b.per_cu, left = wgs % cap;
-            double t = (double)(wgs / cap) * (nsl * (b.per_cu * b.slice + b.load) + b.fixed);
-            if (left)
-                t += nsl * ((left > kNumCUs ? b.per_cu : 1) * b.slice + b.load * left / cap) + b.fixed;
+            double t = kFirst + kNext * (double)((wgs - 1) / cap) +
+                       (double)(wgs / cap) * nsl * (b.per_cu * b.slice + b.load);
+            if (left) t += nsl * ((left > kNumCUs ? b.per_cu : 1) * b.slice + b.load * left / cap);
             const double bytes = (2.0 * p.K * p.N + 2.0 * p.M * p.K +
                                   (p.out_type == kOutF32 ? 4.0 : 2.0) * p.M * p.N) * p.G;
-            t = std::max(t, bytes / 5.9e6 + b.fixed);
+            t = std::max(t, bytes / (5.9e6 * std::min(1.0, (double)wgs / 192)) + kFirst);
             if (split > 1) t += 4.0 * (split + 1) * p.M * p.N * p.G / 3.7e6;
             if (t < best * 0.999) {
                 best = t;

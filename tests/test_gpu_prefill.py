@@ -87,6 +87,9 @@ def gemm_inputs(M, N, K, dt):
     (1332, 1536, 512, "128,128,2"),  # many row tiles, the last of 52 rows
     (130, 392, 224, "128,128,1"),
     (2100, 512, 64, "256,256,1"),    # past one group of eight row tiles
+    (4200, 4104, 64, "256,256,1"),   # 289 tiles on 256 workgroups, the last columns' chunk alone
+    (2000, 9000, 160, "256,128,1"),  # 568 tiles, slices fewer than stages
+    (3300, 4104, 32, "128,128,2"),   # 858 tiles on 512 workgroups (one slice: one split)
 ])
 def test_large_tile_gemm(ext, monkeypatch, dt, M, N, K, plan):
     """Forced large-tile plans against the float64 product of the same 16-bit values (fp32
@@ -109,7 +112,8 @@ def test_16bit_products_by_rule(ext, M, N, K):
 
 
 @pytest.mark.parametrize("dt", [BF, H16], ids=["bf16", "f16"])
-@pytest.mark.parametrize("B,Sq,per_seq", [(5, 26, True), (3, 87, False), (150, 2, True)])
+@pytest.mark.parametrize("B,Sq,per_seq", [(5, 26, True), (3, 87, False), (150, 2, True),
+                                           (265, 2, True)])
 def test_q_absorbed_many_rows(ext, monkeypatch, dt, B, Sq, per_seq):
     """2a2 on the large tiles with 2b in its epilogue, and 2c from its 16-bit q_nope on them:
     the same bits as 2a2, the 2b launch and 2c on the tiled engine from fp32 q_raw
@@ -138,7 +142,7 @@ def test_q_absorbed_many_rows(ext, monkeypatch, dt, B, Sq, per_seq):
 
 
 @pytest.mark.parametrize("dt", [BF, H16], ids=["bf16", "f16"])
-@pytest.mark.parametrize("B,Sq", [(260, 1), (2, 130), (300, 2)])
+@pytest.mark.parametrize("B,Sq", [(260, 1), (2, 130), (300, 2), (7, 100)])
 def test_out_projection_many_rows(ext, monkeypatch, dt, B, Sq):
     """3d on the large tiles (NT, G = heads) gives the tiled engine's bits (MLA_WGEMM=0)."""
     args = [gpu(t) for t in C.attn_inputs(B, Sq, 140, seed=B, dt=dt)]
