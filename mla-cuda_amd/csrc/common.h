@@ -5,6 +5,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 #include "gpu_shape.h"
 
 namespace mla {
@@ -71,6 +73,20 @@ __device__ __forceinline__ float wave_reduce(float v, Op op) {
     const float lo = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 0));
     const float hi = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 32));
     return op(lo, hi);
+}
+
+// Sum of an int over the wave, wave-uniform (the same steps).
+__device__ __forceinline__ int wave_sum(int v) {
+    auto add = [&](auto ctrl) __attribute__((always_inline)) {
+        v += __builtin_amdgcn_update_dpp(0, v, decltype(ctrl)::value, 0xF, 0xF, true);
+    };
+    add(std::integral_constant<int, 0xB1>{});
+    add(std::integral_constant<int, 0x4E>{});
+    add(std::integral_constant<int, 0x141>{});
+    add(std::integral_constant<int, 0x140>{});
+    const auto r = __builtin_amdgcn_permlane16_swap((unsigned)v, (unsigned)v, false, false);
+    v = (int)(r[0] + r[1]);
+    return __builtin_amdgcn_readlane(v, 0) + __builtin_amdgcn_readlane(v, 32);
 }
 
 // A wave-uniform read of kernel-lifetime read-only data (sequence lengths, page tables):

@@ -2630,7 +2630,9 @@ __global__ void __launch_bounds__(kWlThreads) flash_worklist_kernel(const int* _
     // decode step's critical path
     static_assert(kWlThreads == 256 && kWlBuckets == 256, "one bucket per thread, four waves");
     __shared__ long long w_tot[4];
-    __shared__ int w_min[4], w_max[4], w_cnt[4], w_full[4], w_rem[4], w_try[4][kWlTries], w_small[4][kWlTries];
+    __shared__ int w_min[4], w_max[4], w_cnt[4], w_full[4], w_rem[4], w_packs[kWlTries];
+    constexpr int kLdsLens = 1024;   // lengths also kept in LDS, for every wave's candidates
+    __shared__ int s_len[kLdsLens];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int b0 = wl_thread_first(tid, B), b1 = wl_thread_first(tid + 1, B);
     // a thread's lengths stay in registers (up to 8 batches per thread, B <= 2048); past
@@ -2653,6 +2655,7 @@ __global__ void __launch_bounds__(kWlThreads) flash_worklist_kernel(const int* _
     int mn = 0x7fffffff, mx = 0;
     for (int b = b0; b < b1; ++b) {
         const int L = len_of(b);
+        if (b < kLdsLens) s_len[b] = L;
         tot += L;
         mn = min(mn, L);
         mx = max(mx, L);
@@ -2671,30 +2674,25 @@ __global__ void __launch_bounds__(kWlThreads) flash_worklist_kernel(const int* _
     if (mn == mx) {
         chunk = dense_keys_per_split(wl_max(1, mx), B * row_tiles, block_keys);
     } else {
-        // every candidate's piece count in one pass; all threads then pick the same one
+        // wave w tries candidates 2w and 2w + 1 over all batches; the first that packs is taken
         const int base = wl_base_blocks(tot, row_tiles, block_keys);
+        static_assert(kWlTries == 8, "two candidates a wave");
         #pragma unroll
-        for (int k = 0; k < kWlTries; ++k) {
-            const int c = wl_try(base, k, Sk, block_keys);
+        for (int i = 0; i < 2; ++i) {
+            const int c = wl_try(base, 2 * wave + i, Sk, block_keys);
             int n = 0, small = 0;
-            for (int b = b0; b < b1; ++b) {
-                const int L = len_of(b);
+            for (int b = lane; b < B; b += 64) {
+                const int L = b < kLdsLens ? s_len[b] : wl_len(seq_lens[b], Sk);
                 n += wl_chunk_count(L, c);
                 small += wl_small(L, c, block_keys);
             }
-            for (int d = 32; d > 0; d >>= 1) {
-                n += __shfl_xor(n, d);
-                small += __shfl_xor(small, d);
-            }
-            if (lane == 0) { w_try[wave][k] = n; w_small[wave][k] = small; }
+            n = wave_sum(n);
+            small = wave_sum(small);
+            if (lane == 0) w_packs[2 * wave + i] = wl_packs(n, small, tot, c, row_tiles, block_keys);
         }
         __syncthreads();
         int k = 0;
-        for (; k < kWlTries - 1; ++k) {
-            long long n = 0, small = 0;
-            for (int w = 0; w < 4; ++w) { n += w_try[w][k]; small += w_small[w][k]; }
-            if (wl_packs(n, small, tot, wl_try(base, k, Sk, block_keys), row_tiles, block_keys)) break;
-        }
+        while (k < kWlTries - 1 && !w_packs[k]) ++k;
         chunk = wl_try(base, k, Sk, block_keys);
     }
     int cnt, full;

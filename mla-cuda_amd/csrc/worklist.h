@@ -127,13 +127,13 @@ MLA_HD int wl_bucket(int L, int chunk) {
 constexpr int kWlTries = 8;
 MLA_HD int wl_fixed_blocks(int block_keys) { return block_keys == 16 ? 4 : 11; }
 MLA_HD int wl_base_blocks(long long tot, int row_tiles, int block_keys) {
-    const long long per = (tot * row_tiles + kNumCUs - 1) / kNumCUs;
-    const long long blocks = (per + block_keys - 1) / block_keys;
+    const long long per = (tot * row_tiles + kNumCUs - 1) / kNumCUs;   // constants: no division
+    const long long blocks = block_keys == 16 ? (per + 15) / 16 : (per + 31) / 32;
     return blocks < 4 ? 4 : blocks > 0x3fffffff ? 0x3fffffff : (int)blocks;
 }
 // Keys of candidate k: at most the key span rounded up to a block, at least 4 blocks.
 MLA_HD int wl_try(int base_blocks, int k, int Sk, int block_keys) {
-    const int cap = wl_max((Sk + block_keys - 1) / block_keys, 4);
+    const int cap = wl_max(block_keys == 16 ? (Sk + 15) / 16 : (Sk + 31) / 32, 4);
     if (base_blocks >= cap)
         return (block_keys == 16 ? wl_max(4, wl_min(cap, (base_blocks + 3) / 4)) : cap) * block_keys;
     const long long blocks = ((long long)base_blocks * (16 + k) + 15) / 16;
@@ -148,9 +148,9 @@ MLA_HD bool wl_packs(long long pieces, long long small, long long tot, int chunk
                      int block_keys) {
     const long long left = pieces * row_tiles - kNumCUs;
     if (left <= 0) return true;
-    const long long f = wl_fixed_blocks(block_keys);
+    const long long f = wl_fixed_blocks(block_keys) * block_keys;   // all in keys: no division
     return small * row_tiles >= left &&
-           100 * (pieces * f + tot / block_keys) * row_tiles <= 96LL * kNumCUs * (f + chunk / block_keys);
+           100 * (pieces * f + tot) * row_tiles <= 96LL * kNumCUs * (f + chunk);
 }
 
 // The list must fit max_items (the partial slots and the grid are sized for it).  A chunk

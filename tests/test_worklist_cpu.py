@@ -168,5 +168,5 @@ def test_ragged_chunk_packs_or_is_the_last_candidate(block_keys, B, lo, hi):
         short = [int(l) % chunk for l in lens if int(l) % chunk]
         small = sum(2 * s <= chunk - fixed * block_keys for s in short)
         assert n * rt <= 256 or (small * rt >= n * rt - 256 and
-                                 (n * fixed + int(lens.sum()) // block_keys) * rt
-                                 <= 0.96 * 256 * (fixed + chunk // block_keys))
+                                 (n * fixed * block_keys + int(lens.sum())) * rt
+                                 <= 0.96 * 256 * (fixed * block_keys + chunk))
