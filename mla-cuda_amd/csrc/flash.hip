@@ -1978,25 +1978,23 @@ __global__ void __launch_bounds__(kXThreads, 1) flash32x_kernel(FlashArgs a) {
     if (wave < 4) {
         // ================================ score waves
         const int lim_wave = __builtin_amdgcn_readfirstlane(lim);
-        const float* qa = reinterpret_cast<const float*>(a.qa);
-        const float* qr = reinterpret_cast<const float*>(a.qr);
-        const __amdgpu_buffer_rsrc_t rq = make_rsrc(qa + (int64_t)b * rows_b * kFR);
-        const __amdgpu_buffer_rsrc_t rr = make_rsrc(qr + (int64_t)b * rows_b * kFD);
-        const uint32_t qmask = oob_mask(row, rows_b);
-        v4u qf[k32LatReads + k32PeReads];
-        #pragma unroll
-        for (int r = 0; r < k32LatReads; ++r)
-            qf[r] = load16(rq, ((uint32_t)row * (kFR * 4) + 512u * g + 16u * r) | qmask);
-        #pragma unroll
-        for (int r = 0; r < k32PeReads; ++r)
-            qf[k32LatReads + r] = load16(rr, ((uint32_t)row * k32PeBytes + 64u * g + 16u * r) | qmask);
-        wait_vm<0>();   // Q in registers
-
         uint32_t k_base = lat0 + l16 * k32Pitch + 512u * g;   // + stage * k32LatStage
         uint32_t p_off[k32PeReads];
         #pragma unroll
         for (int r = 0; r < k32PeReads; ++r)
             p_off[r] = l16 * k32PeBytes + 16u * ((4 * g + r) ^ swz(l16));
+        v4u qf[k32LatReads + k32PeReads];
+        if (nb > 0) {
+            // Q: this wave's 16 query rows lie in ring stage pw like a block's keys
+            lds_barrier();   // Q: the P.V waves' query loads have landed
+            #pragma unroll
+            for (int r = 0; r < k32LatReads; ++r)
+                qf[r] = *reinterpret_cast<const v4u*>(smem + k_base + (uint32_t)pw * k32LatStage + 16u * r);
+            #pragma unroll
+            for (int r = 0; r < k32PeReads; ++r)
+                qf[k32LatReads + r] = *reinterpret_cast<const v4u*>(smem + (uint32_t)pw * k32PeStage + p_off[r]);
+            lds_barrier();   // Q2: the queries are in registers, the ring is free
+        }
         float m_ref = -INFINITY, m_neg = 0.f, thr = -INFINITY, l_run = 0.f;
         for (int pass = 1;; ++pass) {
             l_run = 0.f;
@@ -2115,6 +2113,33 @@ __global__ void __launch_bounds__(kXThreads, 1) flash32x_kernel(FlashArgs a) {
             dma16_imm<0>(d.rp, d.st_pe, pe_lane);
         }
     };
+    // The tile's queries, in rows of 2 KB like the keys, through the whole ring: wave pw loads
+    // rows 16pw .. +15 into stage pw, where its score wave reads them in the K fragments' pattern;
+    // the first blocks follow into the freed stages.  From global memory straight into those
+    // fragments the 147 KB came in 16-byte pieces, 64 lines an instruction.
+    if (nb > 0) {
+        const uint32_t rows_q = (uint32_t)max(0, min(16, rows_b - r0 - 16 * pw));
+        const int64_t row0 = (int64_t)b * rows_b + min(r0 + 16 * pw, rows_b - 1);
+        const v4i rq = rsrc_span(reinterpret_cast<uint64_t>(reinterpret_cast<const float*>(a.qa) + row0 * kFR),
+                                 0, rows_q * (kFR * 4));
+        const v4i rr = rsrc_span(reinterpret_cast<uint64_t>(reinterpret_cast<const float*>(a.qr) + row0 * kFD),
+                                 0, rows_q * k32PeBytes);
+        const uint32_t ql = __builtin_amdgcn_readfirstlane(lds0 + NS * k32PeStage + pw * k32LatStage);
+        const uint32_t qp = __builtin_amdgcn_readfirstlane(lds0 + pw * k32PeStage);
+        #pragma unroll
+        for (int q = 0; q < 16; ++q) {
+            dma16_imm<0>(rq, ql + q * k32Pitch, 16u * lane + (uint32_t)q * (kFR * 4));
+            dma16_imm<1024>(rq, ql + q * k32Pitch, 16u * lane + (uint32_t)q * (kFR * 4));
+        }
+        #pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const int r = 4 * q + (lane >> 4);
+            dma16_imm<0>(rr, qp + q * 4 * k32PeBytes, (uint32_t)r * k32PeBytes + 16u * ((lane & 15) ^ swz(r)));
+        }
+        wait_vm<0>();
+        lds_barrier();   // Q
+        lds_barrier();   // Q2
+    }
     uint32_t v_base = lat0 + 4 * g * k32Pitch + 8u * l16;   // + stage * k32LatStage
     typedef uint32_t v2u __attribute__((ext_vector_type(2)));
     v4f O[2 * 16];   // [mh][r]
@@ -2178,21 +2203,31 @@ __global__ void __launch_bounds__(kXThreads, 1) flash32x_kernel(FlashArgs a) {
         if (!again) break;
     }
     lds_barrier();       // F
-    // ---- partial state: lane l holds row l%16, columns 32mh + 8g + 2i + r of O[mh][r][i]
-    if (row < rows_b) {
-        const int64_t slot = (work.direct ? (int64_t)b : work.slot) * rows_b + row;
-        if (g == 0) {
-            if (!work.direct) a.m[slot] = xm[16 * pw + l16];
-            (work.direct ? a.l_direct : a.l)[slot] = xl[16 * pw + l16];
-        }
-        float* orow = (work.direct ? a.o_direct : a.o) + slot * kFR;
-        #pragma unroll
-        for (int mh = 0; mh < 16; ++mh) {
-            const v4f lo = {O[2 * mh][0], O[2 * mh + 1][0], O[2 * mh][1], O[2 * mh + 1][1]};
-            const v4f hi = {O[2 * mh][2], O[2 * mh + 1][2], O[2 * mh][3], O[2 * mh + 1][3]};
-            *reinterpret_cast<v4f*>(orow + 32 * mh + 8 * g) = lo;
-            *reinterpret_cast<v4f*>(orow + 32 * mh + 8 * g + 4) = hi;
-        }
+    // ---- partial state: lane l holds row l%16, columns 32mh + 8g + 2i + r of O[mh][r][i].  The
+    // rows go out through this wave's part of the ring (2 KB each, 16-byte chunk c of row r at
+    // c ^ r: writes and reads touch all banks evenly) in 1 KB stores; straight from the registers
+    // a store was 64 pieces of 16 bytes.
+    const int64_t slot0 = (work.direct ? (int64_t)b : work.slot) * rows_b + r0 + 16 * pw;
+    const int rows = rows_b - r0 - 16 * pw;   // of this wave, if below 16
+    if (g == 0 && l16 < rows) {
+        if (!work.direct) a.m[slot0 + l16] = xm[16 * pw + l16];
+        (work.direct ? a.l_direct : a.l)[slot0 + l16] = xl[16 * pw + l16];
+    }
+    uint8_t* const mine = smem + pw * (16 * kFR * 4);
+    #pragma unroll
+    for (int mh = 0; mh < 16; ++mh) {
+        const v4f lo = {O[2 * mh][0], O[2 * mh + 1][0], O[2 * mh][1], O[2 * mh + 1][1]};
+        const v4f hi = {O[2 * mh][2], O[2 * mh + 1][2], O[2 * mh][3], O[2 * mh + 1][3]};
+        *reinterpret_cast<v4f*>(mine + l16 * (kFR * 4) + 16 * ((8 * mh + 2 * g) ^ l16)) = lo;
+        *reinterpret_cast<v4f*>(mine + l16 * (kFR * 4) + 16 * ((8 * mh + 2 * g + 1) ^ l16)) = hi;
+    }
+    __builtin_amdgcn_wave_barrier();
+    float* const dst = (work.direct ? a.o_direct : a.o) + slot0 * kFR + 4 * lane;
+    #pragma unroll
+    for (int q = 0; q < 32; ++q) {
+        const int r = q >> 1;
+        const v4f v = *reinterpret_cast<const v4f*>(mine + r * (kFR * 4) + 16 * ((64 * (q & 1) + lane) ^ r));
+        if (r < rows) *reinterpret_cast<v4f*>(dst + (int64_t)r * kFR + 256 * (q & 1)) = v;
     }
 }
 
