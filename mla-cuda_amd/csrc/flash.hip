@@ -2538,6 +2538,7 @@ constexpr int kFStages = 4;   // LDS ring depth
 // one list read per workgroup: one workgroup per row took 45 us to find the 170,496 rows of a
 // prefill chunk's four sequences already written.
 constexpr int kMergeFew = 8;
+constexpr int kMergeManyRows = kNumCUs / 2;   // up to here flash_merge_many_kernel
 template <int OUT>
 __global__ void __launch_bounds__(256) flash_merge_kernel(const float* __restrict__ o,
                                                           const float* __restrict__ m,
@@ -2648,6 +2649,88 @@ __global__ void __launch_bounds__(256) flash_merge_kernel(const float* __restric
             ls += w * l[slot];
         }
         store(r, acc0, acc1, ls);
+    }
+}
+
+// The merge where a workgroup per row would leave half the CUs idle (kMergeManyRows: one sequence
+// of 128 heads, its keys in up to 256 splits): two workgroups a row (256 columns each, a lane 4 of
+// them), eight waves over the splits (wave w: w, w + 8, ...), their weights ready in LDS so that a
+// wave's loads go out eight at a time; the eight sums are added in wave order.  128 rows of 128
+// splits (33.5 MB): 8.6 us against 13.8.  With more rows its barriers cost more than they give
+// (1,024 rows of 16 splits 14.5 us against 8.0; 256 of 64, attention with 3d, 44.1 against 42.7).
+constexpr int kMergeWeights = 512;
+template <int OUT>
+__global__ void __launch_bounds__(512) flash_merge_many_kernel(const float* __restrict__ o,
+                                                               const float* __restrict__ m,
+                                                               const float* __restrict__ l,
+                                                               void* __restrict__ ctx,
+                                                               float* __restrict__ row_sum, int B,
+                                                               int rows_b, int n_split,
+                                                               const int* __restrict__ wl) {
+    __shared__ float weight[kMergeWeights], red[8], lred[8];
+    __shared__ v4f part[8][64];
+    const int r = blockIdx.x >> 1, half = blockIdx.x & 1;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int b = r / rows_b, i = r - b * rows_b;
+    int64_t unit0 = b, step = B;
+    if (wl) {
+        n_split = load_uniform(wl + kWlHead + B + b);
+        if (n_split == 1) return;
+        unit0 = load_uniform(wl + kWlHead + b);
+        step = 1;
+    }
+    auto slot_of = [&](int s) { return (unit0 + s * step) * rows_b + i; };
+    float mx = -INFINITY;
+    for (int s = tid; s < n_split; s += 512) mx = fmaxf(mx, m[slot_of(s)]);
+    mx = wave_reduce(mx, OpMax{});
+    if (lane == 0) red[wave] = mx;
+    __syncthreads();
+    mx = red[0];
+    #pragma unroll
+    for (int w = 1; w < 8; ++w) mx = fmaxf(mx, red[w]);
+    auto weight_of = [&](int s) {
+        const float ms = m[slot_of(s)];
+        return ms == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(ms - mx);
+    };
+    float ls = 0.f;
+    for (int s = tid; s < n_split; s += 512) {
+        const float w = weight_of(s);
+        if (s < kMergeWeights) weight[s] = w;
+        ls += w * l[slot_of(s)];
+    }
+    ls = wave_reduce(ls, OpSum{});
+    if (lane == 0) lred[wave] = ls;
+    __syncthreads();
+    ls = 0.f;
+    #pragma unroll
+    for (int w = 0; w < 8; ++w) ls += lred[w];
+    v4f acc = {0.f, 0.f, 0.f, 0.f};
+    const float* const col = o + 256 * half + 4 * lane;
+    int s = wave;
+    for (; s + 56 < n_split && s + 56 < kMergeWeights; s += 64) {
+        v4f v[8];
+        #pragma unroll
+        for (int k = 0; k < 8; ++k) v[k] = *reinterpret_cast<const v4f*>(col + slot_of(s + 8 * k) * kFR);
+        #pragma unroll
+        for (int k = 0; k < 8; ++k) acc += weight[s + 8 * k] * v[k];
+    }
+    for (; s < n_split; s += 8)
+        acc += (s < kMergeWeights ? weight[s] : weight_of(s)) *
+               *reinterpret_cast<const v4f*>(col + slot_of(s) * kFR);
+    part[wave][lane] = acc;
+    __syncthreads();
+    if (wave) return;
+    #pragma unroll
+    for (int w = 1; w < 8; ++w) acc += part[w][lane];
+    const int64_t at = (int64_t)r * kFR + 256 * half + 4 * lane;
+    if constexpr (OUT == kOutF32) {
+        *reinterpret_cast<v4f*>(static_cast<float*>(ctx) + at) = acc;
+        if (half == 0 && lane == 0) row_sum[r] = ls;
+    } else {
+        using S = Store16<OUT>;
+        const v4f w = acc * (ls == 0.f ? 0.f : 1.f / ls);
+        *reinterpret_cast<v2u*>(static_cast<uint16_t*>(ctx) + at) = v2u{S::pack2(w[0], w[1]), S::pack2(w[2], w[3])};
     }
 }
 
@@ -3078,10 +3161,24 @@ hipError_t launch_flash(const FlashProblem& p, const FlashPlan& f, float* ctx, f
     hipError_t e = hipGetLastError();
     if (e != hipSuccess || (!f.balanced && f.n_split == 1)) return e;
     if (!merge && !f.balanced) return e;   // the caller folds the merge in
-    // few rows: one per workgroup; many: four, and 64 once that still fills the chip
-    const int rpw = rows <= 2048 ? 1 : rows < 65536 ? 4 : 64;
-    const dim3 mgrid((unsigned)((rows + rpw - 1) / rpw)), mblock(256);
     const int n = f.n_split;
+    if (rows <= kMergeManyRows) {
+        const dim3 grid2((unsigned)(2 * rows)), block2(512);
+        if (!ctx16)
+            hipLaunchKernelGGL(flash_merge_many_kernel<kOutF32>, grid2, block2, 0, stream, a.o, a.m, a.l,
+                               ctx, row_sum, p.B, rows_b, n, a.wl);
+        else if (p.f16)
+            hipLaunchKernelGGL(flash_merge_many_kernel<kOutF16>, grid2, block2, 0, stream, a.o, a.m, a.l,
+                               ctx16, nullptr, p.B, rows_b, n, a.wl);
+        else
+            hipLaunchKernelGGL(flash_merge_many_kernel<kOutBF16>, grid2, block2, 0, stream, a.o, a.m, a.l,
+                               ctx16, nullptr, p.B, rows_b, n, a.wl);
+        return hipGetLastError();
+    }
+    // few rows: one per workgroup; many: four (a wave each); a large list's, whose batches mostly
+    // need no merge: 64, so that finding that out takes fewer workgroups
+    const int rpw = rows <= 2048 ? 1 : f.balanced && rows >= 65536 ? 64 : 4;
+    const dim3 mgrid((unsigned)((rows + rpw - 1) / rpw)), mblock(256);
     if (!ctx16)
         hipLaunchKernelGGL(flash_merge_kernel<kOutF32>, mgrid, mblock, 0, stream, a.o, a.m, a.l, ctx,
                            row_sum, p.B, rows, rows_b, n, rpw, a.wl);

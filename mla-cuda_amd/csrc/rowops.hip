@@ -25,7 +25,8 @@ constexpr int kNormCache = 4;  // float4 per thread kept in registers (256*4*4 =
 
 // Sum of nsplit partial rows (slice order) at float4 column c4.  NS > 0: nsplit == NS,
 // known at compile time, and all NS loads are issued before the first add (one memory
-// latency instead of one per batch); the additions run in the same order either way.
+// latency instead of one per batch); NS < 0: the same for any nsplit <= -NS, the others'
+// places zeros; the additions run in the same order in every form.
 template <int NS = 0>
 __device__ __forceinline__ v4f sum_partials4(const float* base, int nsplit, int64_t split_stride,
                                              int c4) {
@@ -36,6 +37,18 @@ __device__ __forceinline__ v4f sum_partials4(const float* base, int nsplit, int6
         v4f v = p[0];
         #pragma unroll
         for (int s = 1; s < NS; ++s) v += p[s];
+        return v;
+    }
+    if constexpr (NS < 0) {
+        v4f p[-NS];
+        #pragma unroll
+        for (int s = 0; s < -NS; ++s)
+            p[s] = s < nsplit ? *reinterpret_cast<const v4f*>(base + s * split_stride + 4 * c4)
+                              : v4f{0.f, 0.f, 0.f, 0.f};
+        v4f v = p[0];
+        #pragma unroll
+        for (int s = 1; s < -NS; ++s)
+            if (s < nsplit) v += p[s];
         return v;
     }
     v4f v = *reinterpret_cast<const v4f*>(base + 4 * c4);
@@ -264,7 +277,7 @@ __global__ void __launch_bounds__(256) stream_merge_kernel(float* __restrict__ c
 // columns rotated exactly as 2b rotates, and both land in cache row start_row + s of
 // batch b.  The input is the GEMM output x @ W_kv_a or its nsplit split-K partials, rows
 // of ld = kv_rank + rope floats; partials are summed in slice order.
-template <int OUT>
+template <int OUT, int NS>
 __global__ void __launch_bounds__(256) kv_append_kernel(const float* __restrict__ in, int nsplit,
                                                         int64_t split_stride, const void* gain,
                                                         const int64_t* __restrict__ positions,
@@ -289,13 +302,24 @@ __global__ void __launch_bounds__(256) kv_append_kernel(const float* __restrict_
     } else {
         crow = (int64_t)b * cache_rows + start_row + s;
     }
-    // rope pairs first (no barrier inside), then the workgroup-wide norm
-    for (int i = threadIdx.x; i < D / 2; i += blockDim.x) {
-        float x0 = base[R + 2 * i], x1 = base[R + 2 * i + 1];
-        for (int q = 1; q < nsplit; ++q) {
-            x0 += base[q * split_stride + R + 2 * i];
-            x1 += base[q * split_stride + R + 2 * i + 1];
+    // rope pairs first (no barrier inside), then the workgroup-wide norm.  The pairs are the last
+    // threads': at the cache's widths (R = 512, D = 64) the norm's loads are the first 128's, so
+    // both wait for their partials at the same time.
+    for (int i = 255 - (int)threadIdx.x; i < D / 2; i += 256) {
+        typedef float v2f __attribute__((ext_vector_type(2)));
+        auto pair = [&](int q) { return *reinterpret_cast<const v2f*>(base + q * split_stride + R + 2 * i); };
+        v2f x = pair(0);
+        if constexpr (NS < 0) {
+            v2f p[-NS];
+            #pragma unroll
+            for (int q = 1; q < -NS; ++q) p[q] = q < nsplit ? pair(q) : v2f{0.f, 0.f};
+            #pragma unroll
+            for (int q = 1; q < -NS; ++q)
+                if (q < nsplit) x += p[q];
+        } else {
+            for (int q = 1; q < nsplit; ++q) x += pair(q);
         }
+        const float x0 = x[0], x1 = x[1];
         const float ang = rope_angle(pos, inv_freq[i]);
         float c, sn;
         rope_cos_sin(ang, &c, &sn);
@@ -311,7 +335,7 @@ __global__ void __launch_bounds__(256) kv_append_kernel(const float* __restrict_
     void* out_row = OUT == kOutF32
                         ? static_cast<void*>(static_cast<float*>(c_kv) + crow * R)
                         : static_cast<void*>(static_cast<uint16_t*>(c_kv) + crow * R);
-    rms_row<OUT>(base, nsplit, split_stride, gain, out_row, R, eps, red);
+    rms_row<OUT, NS>(base, nsplit, split_stride, gain, out_row, R, eps, red);
 }
 
 // ---- fp8 cache decoding: out[i] = code[i] * scale, OCP e4m3 codes, through the same
@@ -755,21 +779,17 @@ hipError_t launch_kv_append(const float* in, int nsplit, int64_t split_stride, c
     const int64_t rows = (int64_t)B * Sq;
     if (rows <= 0) return hipSuccess;
     if (rows > 0x7fffffff) return hipErrorInvalidValue;
-    if (out_type == kOutF32)
-        hipLaunchKernelGGL(kv_append_kernel<kOutF32>, dim3((unsigned)rows), dim3(256), 0, stream,
-                           in, nsplit, split_stride, gain, positions, inv_freq, c_kv, pe, Sq, R,
-                           D, start_row, cache_rows, pos_per_batch ? 1 : 0, block_table,
-                           page_size, max_pages, eps);
-    else if (out_type == kOutBF16)
-        hipLaunchKernelGGL(kv_append_kernel<kOutBF16>, dim3((unsigned)rows), dim3(256), 0, stream,
-                           in, nsplit, split_stride, gain, positions, inv_freq, c_kv, pe, Sq, R,
-                           D, start_row, cache_rows, pos_per_batch ? 1 : 0, block_table,
-                           page_size, max_pages, eps);
-    else
-        hipLaunchKernelGGL(kv_append_kernel<kOutF16>, dim3((unsigned)rows), dim3(256), 0, stream,
-                           in, nsplit, split_stride, gain, positions, inv_freq, c_kv, pe, Sq, R,
-                           D, start_row, cache_rows, pos_per_batch ? 1 : 0, block_table,
-                           page_size, max_pages, eps);
+    // up to 16 split partials, and no more rows than CUs: all a row's loads at once (8 rows of 14
+    // splits 8.2 -> 5.1 us; with many rows its registers cost more, 1,332 rows 7.3 -> 10.0)
+    auto launch = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3((unsigned)rows), dim3(256), 0, stream, in, nsplit, split_stride,
+                           gain, positions, inv_freq, c_kv, pe, Sq, R, D, start_row, cache_rows,
+                           pos_per_batch ? 1 : 0, block_table, page_size, max_pages, eps);
+    };
+    const bool few = nsplit > 1 && nsplit <= 16 && rows <= kNumCUs;
+    if (out_type == kOutF32) few ? launch(kv_append_kernel<kOutF32, -16>) : launch(kv_append_kernel<kOutF32, 0>);
+    else if (out_type == kOutBF16) few ? launch(kv_append_kernel<kOutBF16, -16>) : launch(kv_append_kernel<kOutBF16, 0>);
+    else few ? launch(kv_append_kernel<kOutF16, -16>) : launch(kv_append_kernel<kOutF16, 0>);
     return hipGetLastError();
 }
 
