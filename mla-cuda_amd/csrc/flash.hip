@@ -1972,6 +1972,11 @@ __global__ void __launch_bounds__(kXThreads, 1) flash32x_kernel(FlashArgs a) {
         k_hi = min(k_hi, skb - a.Sq + min(r0 + kFRows - 1, rows_b - 1) / a.H + 1);
     }
     const int nb = k_hi > k_lo ? (k_hi - k_lo + k32Keys - 1) / k32Keys : 0;
+    // Queries through the ring where workgroups follow one another on a CU: 8,192 tiles of B=8
+    // S=512 take 2,393 us so, 2,429 us with each score wave loading its own.  A grid that starts
+    // all at once loads them directly, beside the first blocks, which the ring makes wait: B=128
+    // Sk=4989 1,240 us so, 1,243 us through the ring.
+    const bool q_ring = gridDim.x > kNumCUs;
     const uint32_t lat0 = NS * k32PeStage;
     const uint32_t pslot = kPBase + pw * 1024 + 16u * lane;   // + stage * k32XPStage
 
@@ -1984,7 +1989,20 @@ __global__ void __launch_bounds__(kXThreads, 1) flash32x_kernel(FlashArgs a) {
         for (int r = 0; r < k32PeReads; ++r)
             p_off[r] = l16 * k32PeBytes + 16u * ((4 * g + r) ^ swz(l16));
         v4u qf[k32LatReads + k32PeReads];
-        if (nb > 0) {
+        if (!q_ring) {
+            const float* qa = reinterpret_cast<const float*>(a.qa);
+            const float* qr = reinterpret_cast<const float*>(a.qr);
+            const __amdgpu_buffer_rsrc_t rq = make_rsrc(qa + (int64_t)b * rows_b * kFR);
+            const __amdgpu_buffer_rsrc_t rr = make_rsrc(qr + (int64_t)b * rows_b * kFD);
+            const uint32_t qmask = oob_mask(row, rows_b);
+            #pragma unroll
+            for (int r = 0; r < k32LatReads; ++r)
+                qf[r] = load16(rq, ((uint32_t)row * (kFR * 4) + 512u * g + 16u * r) | qmask);
+            #pragma unroll
+            for (int r = 0; r < k32PeReads; ++r)
+                qf[k32LatReads + r] = load16(rr, ((uint32_t)row * k32PeBytes + 64u * g + 16u * r) | qmask);
+            wait_vm<0>();   // Q in registers
+        } else if (nb > 0) {
             // Q: this wave's 16 query rows lie in ring stage pw like a block's keys
             lds_barrier();   // Q: the P.V waves' query loads have landed
             #pragma unroll
@@ -2116,8 +2134,8 @@ __global__ void __launch_bounds__(kXThreads, 1) flash32x_kernel(FlashArgs a) {
     // The tile's queries, in rows of 2 KB like the keys, through the whole ring: wave pw loads
     // rows 16pw .. +15 into stage pw, where its score wave reads them in the K fragments' pattern;
     // the first blocks follow into the freed stages.  From global memory straight into those
-    // fragments the 147 KB came in 16-byte pieces, 64 lines an instruction.
-    if (nb > 0) {
+    // fragments the 147 KB come in 16-byte pieces, 64 lines an instruction.
+    if (q_ring && nb > 0) {
         const uint32_t rows_q = (uint32_t)max(0, min(16, rows_b - r0 - 16 * pw));
         const int64_t row0 = (int64_t)b * rows_b + min(r0 + 16 * pw, rows_b - 1);
         const v4i rq = rsrc_span(reinterpret_cast<uint64_t>(reinterpret_cast<const float*>(a.qa) + row0 * kFR),

@@ -375,3 +375,17 @@ def test_bf16_pv_layouts_same_bits(ext, monkeypatch, B, Sq, Sk, causal):
     monkeypatch.setenv("MLA_FLASH16_PV", "32")
     b = run(ext, args, causal)
     assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("dt", [BF, torch.float16, F32], ids=["bf16", "f16", "f32"])
+@pytest.mark.parametrize("B,Sq,H,splits", [(1, 1, 128, 2), (1, 1, 128, 130), (1, 3, 40, 17),
+                                           (1, 3, 43, 17), (16, 1, 8, 9)])
+def test_merge_few_rows(ext, monkeypatch, dt, B, Sq, H, splits):
+    """Merges of at most 128 rows (two workgroups each) and of 129 (a workgroup each): fewer
+    splits than waves, more than a round of them, a last split of 7 keys, and with Sq = 3
+    causal rows that see none of it."""
+    Sk = 32 * (splits - 1) + 7
+    monkeypatch.setenv("MLA_FLASH_SPLITS", str((Sk + 31) // 32))
+    args = inputs(B, Sq, Sk, H=H, seed=Sk + H, dt=dt)
+    got = run(ext, args, Sq > 1).float().cpu()
+    close(got, oracle(args, Sq > 1), dt)

@@ -91,6 +91,22 @@ def test_kv_append_16bit(ext, dtype):
                                **TOL_BF16)
 
 
+@pytest.mark.parametrize("B,split", [(1, 2), (8, 5), (8, 16), (8, 17), (256, 3), (257, 3)])
+def test_kv_append_split_partials(ext, monkeypatch, B, split):
+    """Split partials of x @ W_kv_a summed on load: up to 16 of few rows at once, more of
+    them or of more rows one after the other; the plan is forced, the oracle is the same."""
+    x, W, gain, ck, pe = kv_inputs(B, 1, 3, seed=split)
+    pos = torch.tensor([31 * split + 5])
+    monkeypatch.setenv("MLA_GEMM_PLAN", f"{B},{D.kv_rank + D.rope},{D.hidden},1=64,64,{split}")
+    ck_g, pe_g = gpu(ck), gpu(pe)
+    ext.kv_append(gpu(x), gpu(W), gpu(gain), gpu(pos), ck_g, pe_g, 1, 1e-6)
+    pick = [0, B // 2, B - 1]
+    for b in pick:
+        rc, rp = R.kv_append(x[b:b + 1], W, gain, pos, ck[b:b + 1], pe[b:b + 1], 1, eps=1e-6)
+        torch.testing.assert_close(ck_g[b:b + 1].cpu(), rc, **TOL)
+        torch.testing.assert_close(pe_g[b:b + 1].cpu(), rp, **TOL)
+
+
 def test_kv_append_then_decode(ext):
     """Decode step end to end: append the new token's cache row, then attend over the
     extended cache; the oracle does the same on the CPU."""
