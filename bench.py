@@ -191,8 +191,9 @@ def in_layer_kernel_us(layer, flush, n):
     kernels attributed to steps by launch order -- the layer launches its GEMMs in the order
     2a1, 2a2, 2c, 3d, a split-K reduce right after its GEMM, RMSNorm (2a-n, which also sums
     2a1's split partials) and RoPE (2b) between them (the 16-bit 2a2 may do 2b and 2c in its
-    epilogue: `wgemm_kernel<.., 2, false>`, counted as 2a2; an unsplit fp32 2a2 may do 2b:
-    `gemm_kernel<.., true>`, its last template argument; at decode-sized fp32 batches
+    epilogue: `wgemm_kernel<.., 2, false>`, counted as 2a2; an unsplit fp32 2a2 or a
+    large-tile 16-bit one may do 2b: `gemm_kernel<.., true>`, `bgemm_kernel<.., true>`, the
+    last template argument; at decode-sized fp32 batches
     `q_small_kernel` does 2b and 2c, counted as 2c), and the fused attention's kernels
     (work list, pass, merge) as 3abc; at decode-sized fp32 batches 3d may be
     out_small_kernel, which also does the pass's split merge.  Returns {step: mean µs per
@@ -246,7 +247,7 @@ def attribute_steps(ks):
                 cur["gemm"] += 1      # 2a2 with 2b and 2c in its epilogue: no 2c launch
                 folded["2a2"] = ("2b", "2c")
             elif step == "2a2" and "wgemm_kernel" not in name and re.search(r",\s*true>", name):
-                folded["2a2"] = ("2b",)   # the fp32 2a2 that rotates q_rope in its epilogue
+                folded["2a2"] = ("2b",)   # the 2a2 that rotates q_rope in its epilogue
         elif "split_reduce" in name:
             step = cur["step"] or "2a1"
         elif "rmsnorm" in name:

@@ -18,7 +18,7 @@ namespace mla {
 enum AMode { kAPlain = 0, kARowRecip = 1, kAAlpha = 2 };
 enum OutType { kOutF32 = 0, kOutBF16 = 1, kOutF16 = 2 };   // the codes Store16<> takes
 
-// 2a2's fused epilogue (16-bit weight-streaming plans with split 1 only): instead of the
+// 2a2's fused epilogue (16-bit weight-streaming or large-tile plans with split 1): instead of the
 // fp32 product C [M, H*(nope+rope)], the nope columns of every head go to q_nope
 // [M, H, nope] and the rope columns, rotated, to q_rope [M, H, rope], both rounded once to
 // the storage format -- the rounding 2c and 2b apply to the same fp32 values.  The rotation
@@ -26,7 +26,7 @@ enum OutType { kOutF32 = 0, kOutBF16 = 1, kOutF16 = 2 };   // the codes Store16<
 // 2a-n launch writes (RopeTable).  nope and rope are multiples of 32, rope <= 64.
 // With w_uk set the epilogue also does 2c: each head's 16-bit q_nope tile stays in LDS and
 // is multiplied by W_uk[h] ([H, nope, kv] contiguous) into q_abs [M, H, kv] (storage
-// format), and q_nope is not written.  That needs the 128 x 4 plan, nope = 128, rope = 64,
+// format), and q_nope is not written.  That needs the weight-streaming 128 x 4 plan, nope = 128, rope = 64,
 // an even H and kv a multiple of 128 up to 512 (qup_supported).
 struct QUpEpilogue {
     void* q_nope = nullptr;
@@ -68,7 +68,7 @@ struct GemmProblem {
     const int* k_len = nullptr;
     const int* b_pages = nullptr;
     int page_size = 0, max_pages = 0;
-    const QUpEpilogue* qup = nullptr;   // weight-streaming plans only (launch_wgemm)
+    const QUpEpilogue* qup = nullptr;   // launch_wgemm; launch_bgemm at rope = 64, without w_uk
     // fp32 tiled plans with one K split: 2b in 2a2's epilogue (q_rope, cos_sin, H, nope,
     // rope of the struct; the nope columns still go to C)
     const QUpEpilogue* rope_epi = nullptr;
