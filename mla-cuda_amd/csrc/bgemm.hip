@@ -455,7 +455,8 @@ bool bgemm_supported(const GemmProblem& p, int bm, int bn, int split) {
     const OutType own16 = p.f16 ? kOutF16 : kOutBF16;
     return p.half && !p.a_f32 && p.amode == kAPlain && split >= 1 && bgemm_tile(bm, bn) &&
            (p.out_type == kOutF32 || split > 1 || p.out_type == own16) && !p.k_len && !p.b_pages &&
-           p.M > 0 && p.G >= 1 && p.N % 8 == 0 && p.K % kBKS == 0 && p.lda >= kBKS &&
+           p.M > 0 && p.G >= 1 && (p.G == 1 || split == 1) &&   // job_at's order of groups has no splits
+           p.N % 8 == 0 && p.K % kBKS == 0 && p.lda >= kBKS &&
            (p.b_nt ? p.ldb >= p.K : p.ldb >= p.N) &&
            // 16-byte aligned rows and groups, of the operands and of a 16-bit C
            p.lda % 8 == 0 && p.ldb % 8 == 0 && p.sAg % 8 == 0 && p.sBg % 8 == 0 &&

@@ -264,6 +264,21 @@ def test_weight_streaming_plans_size_the_workspace(lib, monkeypatch):
     assert lib.mla_gemm_workspace_bytes(BF16, 40, 200, 128) == tiled
 
 
+@pytest.mark.parametrize("tile", ["256,256", "256,128", "128,128"])
+def test_forced_large_tiles_take_no_grouped_split(lib, monkeypatch, tile):
+    """The large-tile engine splits K of ungrouped products only: MLA_BGEMM_PLAN's split is
+    taken for mla_gemm and ignored for 2c and 3d (a group per head), whose workspaces then are
+    those without the variable."""
+    d = dsv3(200, 1, 4989)
+    q = lambda: lib.mla_q_absorbed_workspace_bytes(BF16, ctypes.byref(d))  # noqa: E731
+    attn = lambda: lib.mla_attention_workspace_bytes(BF16, ctypes.byref(d), 0)  # noqa: E731
+    want = q(), attn()
+    monkeypatch.setenv("MLA_BGEMM_PLAN", f"200,512,128,128={tile},2;200,128,512,128={tile},2;"
+                                         f"200,512,1024,1={tile},2")
+    assert lib.mla_gemm_workspace_bytes(BF16, 200, 512, 1024) == 2 * 200 * 512 * 4
+    assert (q(), attn()) == want
+
+
 def test_attention_validation(lib):
     d = dsv3(2, 3, 2)
     args = [P16] * 5
