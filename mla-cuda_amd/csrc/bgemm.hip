@@ -202,7 +202,7 @@ __global__ void __launch_bounds__(kBThreads, MINB) bgemm_kernel(BArgs a) {
                                          : kAStage + (uint32_t)(wave * kLoadsB + q - kLoadsA) * 1024u;
         uint32_t v = q < kLoadsA ? a_voff[q < kLoadsA ? q : 0] : b_voff[q < kLoadsA ? 0 : q - kLoadsA];
         if constexpr (QUP) v ^= (v ^ (d.tab + off + 16u * lane)) & d.tab_mask;
-        dma16(q < kLoadsA ? d.ra : d.rb, d.st + off, v, 0);
+        dma16(q < kLoadsA ? d.ra : d.rb, d.st + off, v);
     };
 
     // ---- fragments: wave (wm, wn) covers rows (BM/2) wm .. and columns (BN/4) wn ..

@@ -410,11 +410,11 @@ __global__ void __launch_bounds__(kFThreads, 1) flash16_kernel(FlashArgs a) {
     const uint32_t pe8_lane = lane < 32 ? lane16 : kOob;   // 8 rope rows of 64 B: 32 lanes
     auto issue_one = [&](const Loads& d, int q) __attribute__((always_inline)) {
         if constexpr (FP8) {
-            if (q < 4) dma16(d.rk, d.st + q * 1024, lane16, q * 1024);
-            else dma16(d.rp, d.st_pe, pe8_lane, 0);
+            if (q < 4) dma16(d.rk, d.st + q * 1024, lane16 + q * 1024);
+            else dma16(d.rp, d.st_pe, pe8_lane);
         } else {
-            if (q < 8) dma16(d.rk, d.st + q * kLatBytes, lane16 ^ (16u * sw16((8 * wave + q) & 15)), q * kLatBytes);
-            else dma16(d.rp, d.st_pe, pe_lane, 0);
+            if (q < 8) dma16(d.rk, d.st + q * kLatBytes, (lane16 ^ (16u * sw16((8 * wave + q) & 15))) + q * kLatBytes);
+            else dma16(d.rp, d.st_pe, pe_lane);
         }
     };
 
@@ -1073,11 +1073,11 @@ __global__ void __launch_bounds__(kXThreads, 1) flash16x_kernel(FlashArgs a) {
     const uint32_t pe8_lane = lane < 32 ? lane16 : kOob;   // 8 rope rows of 64 B: 32 lanes
     auto issue_one = [&](const Loads& d, int q) __attribute__((always_inline)) {
         if constexpr (FP8) {
-            if (q < 4) dma16(d.rk, d.st + q * 1024, lane16, q * 1024);
-            else dma16(d.rp, d.st_pe, pe8_lane, 0);
+            if (q < 4) dma16(d.rk, d.st + q * 1024, lane16 + q * 1024);
+            else dma16(d.rp, d.st_pe, pe8_lane);
         } else {
-            if (q < 8) dma16(d.rk, d.st + q * kLatBytes, lane16 ^ (16u * sw16((8 * wv + q) & 15)), q * kLatBytes);
-            else dma16(d.rp, d.st_pe, pe_lane, 0);
+            if (q < 8) dma16(d.rk, d.st + q * kLatBytes, (lane16 ^ (16u * sw16((8 * wv + q) & 15))) + q * kLatBytes);
+            else dma16(d.rp, d.st_pe, pe_lane);
         }
     };
     const F8Stage f8(wv, lane, kPeBase);
@@ -1107,12 +1107,11 @@ __global__ void __launch_bounds__(kXThreads, 1) flash16x_kernel(FlashArgs a) {
             const uint32_t qp = __builtin_amdgcn_readfirstlane(lds0 + kPeBase + st * k2PeStage + slot0 * kPeBytes);
             #pragma unroll
             for (int q = 0; q < 16; ++q)
-                dma16(rq, ql + q * kLatBytes, lane16 ^ (16u * sw16(q)), (row0 + q) * kLatBytes);
+                dma16(rq, ql + q * kLatBytes, (lane16 ^ (16u * sw16(q))) + (row0 + q) * kLatBytes);
             #pragma unroll
             for (int q = 0; q < 2; ++q)
                 dma16(rr, qp + q * 1024,
-                      (uint32_t)(lane >> 3) * kPeBytes + 16u * ((lane & 7) ^ ((4 * q + (lane >> 4)) & 7)),
-                      (row0 + 8 * q) * kPeBytes);
+                      (row0 + 8 * q + (lane >> 3)) * kPeBytes + 16u * ((lane & 7) ^ ((4 * q + (lane >> 4)) & 7)));
         }
     }
     v16f O[8];
@@ -1532,8 +1531,8 @@ __global__ void __launch_bounds__(kXThreads, 1) flash16x8_kernel(FlashArgs a) {
         return d;
     };
     auto issue_one = [&](const Loads& d, int q) __attribute__((always_inline)) {
-        if (q < 4) dma16(d.rk, d.st + q * 1024, lat_voff[q], 0);
-        else dma16(d.rp, d.st_pe, pe_voff, 0);
+        if (q < 4) dma16(d.rk, d.st + q * 1024, lat_voff[q]);
+        else dma16(d.rp, d.st_pe, pe_voff);
     };
     // loads per block: 5 for the rope loaders, 4 for the others; wait until at most n
     // blocks' loads are outstanding
@@ -1559,12 +1558,11 @@ __global__ void __launch_bounds__(kXThreads, 1) flash16x8_kernel(FlashArgs a) {
         const uint32_t qp = __builtin_amdgcn_readfirstlane(lds0 + kQBase + kFRows * kLatBytes + row0 * kPeBytes);
         #pragma unroll
         for (int q = 0; q < 16; ++q)
-            dma16(rq, ql + q * kLatBytes, 16u * (lane ^ q), (row0 + q) * kLatBytes);
+            dma16(rq, ql + q * kLatBytes, 16u * (lane ^ q) + (row0 + q) * kLatBytes);
         #pragma unroll
         for (int q = 0; q < 2; ++q)
             dma16(rr, qp + q * 1024,
-                  (uint32_t)(lane >> 3) * kPeBytes + 16u * ((lane & 7) ^ ((4 * q + (lane >> 4)) & 7)),
-                  (row0 + 8 * q) * kPeBytes);
+                  (row0 + 8 * q + (lane >> 3)) * kPeBytes + 16u * ((lane & 7) ^ ((4 * q + (lane >> 4)) & 7)));
     }
     v16f O[8];
     for (int pass = 1;; ++pass) {

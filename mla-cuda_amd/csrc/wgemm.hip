@@ -164,10 +164,11 @@ __global__ void __launch_bounds__(kWThreads, MINB) wgemm_kernel(WArgs a) {
             for (int q = 0; q < kLoadsB; ++q) {
                 const int r = (wave * kLoadsB + q) * kRowsPerLoadB + lane / (kBRow / 16);
                 const int pos = lane % (kBRow / 16);
-                const uint32_t voff = (uint32_t)r * (uint32_t)kv * 2u + 16u * (pos ^ (4 * (r & 3)));
+                const uint32_t voff = (uint32_t)r * (uint32_t)kv * 2u + 16u * (pos ^ (4 * (r & 3))) +
+                                      (live ? (uint32_t)(kh * kWKS * kv * 2 + 256 * p) : 0u);
                 dma16(rw, __builtin_amdgcn_readfirstlane(
                               lds0 + wuk_slot(p, kh) + (uint32_t)((wave * kLoadsB + q) * kRowsPerLoadB) * kBRow),
-                      voff, live ? (uint32_t)(kh * kWKS * kv * 2 + 256 * p) : 0u);
+                      voff);
             }
         }
     };
@@ -189,13 +190,13 @@ __global__ void __launch_bounds__(kWThreads, MINB) wgemm_kernel(WArgs a) {
         #pragma unroll
         for (int q = 0; q < kWLoadsA; ++q)
             dma16(ra, __builtin_amdgcn_readfirstlane(st + (uint32_t)(32 * wave + 8 * q) * 128u),
-                  a_voff[q], 0);
+                  a_voff[q]);
         #pragma unroll
         for (int q = 0; q < kLoadsB; ++q)
             dma16(rb, __builtin_amdgcn_readfirstlane(
                           NT ? st + kWAStage + (uint32_t)((BN / 4) * wave + 8 * q) * 128u
                              : st + kWAStage + (uint32_t)((wave * kLoadsB + q) * kRowsPerLoadB) * kBRow),
-                  b_voff[q], 0);
+                  b_voff[q]);
     };
 
     // ---- fragments: wave (wm, wn) covers rows 64wm .. +63 and columns (BN/2)wn .. +BN/2-1
@@ -264,7 +265,7 @@ __global__ void __launch_bounds__(kWThreads, MINB) wgemm_kernel(WArgs a) {
                                      0, (uint32_t)(rows_a * half * 8));
             for (int b = wave; b < half; b += 4)   // kWBM * half * 8 bytes = half KB
                 dma16(rt, __builtin_amdgcn_readfirstlane(lds0 + NS * kStage + 1024u * b),
-                      1024u * b + 16u * lane, 0);
+                      1024u * b + 16u * lane);
         }
     }
     if constexpr (QUP == kQupAbsorb) {
