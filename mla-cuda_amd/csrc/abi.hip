@@ -224,7 +224,13 @@ GemmProblem q_down_problem(mla_dtype_t dt, const mla_dims_t* d, const void* x, c
     p.B = W; p.ldb = d->q_lora;
     p.C = C; p.ldc = d->q_lora;
     p.M = d->batch * d->sq; p.N = d->q_lora; p.K = d->hidden;
+    p.sums_split = true;   // 2a-n
     return p;
+}
+
+// The head widths that 2a2's fused epilogue takes (qup_fused).
+bool qup_heads(const mla_dims_t* d) {
+    return d->nope % 32 == 0 && d->rope % 32 == 0 && d->rope > 0 && d->rope <= 64;
 }
 
 GemmProblem q_up_problem(mla_dtype_t dt, const mla_dims_t* d, const void* q_lat, const void* W,
@@ -236,6 +242,8 @@ GemmProblem q_up_problem(mla_dtype_t dt, const mla_dims_t* d, const void* q_lat,
     p.B = W; p.ldb = n;
     p.C = C; p.ldc = n;
     p.M = d->batch * d->sq; p.N = n; p.K = d->q_lora;
+    p.sums_split = true;   // 2b
+    if (is_half(dt) && qup_heads(d)) p.fuse_rope = d->rope;
     return p;
 }
 
@@ -304,7 +312,7 @@ bool qup_fused(mla_dtype_t dt, const mla_dims_t* d, const GemmPlan& up) {
     const char* env = getenv("MLA_QUP_FUSE");
     if (env && strcmp(env, "0") == 0) return false;
     return is_half(dt) && ((up.bgemm && d->rope == 64) || (up.wgemm && up.bn <= 128)) && up.split == 1 &&
-           d->nope % 32 == 0 && d->rope % 32 == 0 && d->rope > 0 && d->rope <= 64;
+           qup_heads(d);
 }
 
 // 2a2's fused epilogue with 2c as well (wgemm.hip, qup_supported): one head's nope columns
@@ -590,6 +598,7 @@ GemmProblem kv_problem(mla_dtype_t dt, const mla_dims_t* d, const void* x, const
     p.B = W; p.ldb = n;
     p.C = C; p.ldc = n;
     p.M = d->batch * d->sq; p.N = n; p.K = d->hidden;
+    p.sums_split = true;   // the append
     return p;
 }
 

@@ -725,8 +725,91 @@ bool plan_override(const GemmProblem& p, GemmPlan* out) {
     return false;
 }
 
-// The 16-bit products with 16-bit A run on two engines: up to 128 rows on the weight-streaming
-// one (wgemm.hip), past that on the large-tile one (bgemm.hip).  The line lies at one row tile
+// The tiled engine's plan, from the model above.
+void tiled_rule(const GemmProblem& p, GemmPlan* out) {
+    // fp32 MFMA: 256 flop/clk/CU at 2.4 GHz; dense bf16 MFMA is 16x that
+    const double kCuRate = 256.0 * 2.4e9 * (p.half ? 16.0 : 1.0);
+    constexpr double kHbm = 5.0e12;             // sustained HBM B/s
+    constexpr double kReduceLaunch = 3e-6;      // s
+    const int kBK = p.half ? 64 : 32;           // K per slice
+    const double eb = p.half ? 2.0 : 4.0;       // bytes per B element
+    const double ea = p.a_f32 || !p.half ? 4.0 : 2.0;
+    const int kslices = cdiv(p.K, kBK);
+    double best_t = 1e300;
+    for (const auto& t : kTiles) {
+        const int tm = cdiv(p.M, t.bm), tn = cdiv(p.N, t.bn);
+        const int64_t tiles = (int64_t)tm * tn * p.G;
+        const int occ = std::max(1, std::min(2, 163840 / lds_bytes(t.bm, t.bn, p.b_nt, p.half)));
+        for (int split = 1; split <= std::max(1, kslices / 2); split *= 2) {
+            const int per = cdiv(kslices, split);
+            const int real_split = cdiv(kslices, per);
+            if (real_split != split && split > 1) continue;
+            const int64_t blocks = tiles * split;
+            // the busiest CU runs ceil(blocks / CUs) workgroups back to back or side by
+            // side; a lone workgroup per CU hides latency worse than two
+            const int64_t per_cu = (blocks + kNumCUs - 1) / kNumCUs;
+            const double hide = std::min<int64_t>(per_cu, occ) >= 2 ? 1.0 : 0.8;
+            // a workgroup's first slices and its epilogue are not overlapped with MFMA
+            // work: about four slices' worth of pipeline fill and drain
+            const double fill = per / (per + 4.0);
+            const double wg_flops = 2.0 * t.bm * t.bn * (double)per * kBK;
+            const double t_mfma = per_cu * wg_flops / (kCuRate * t.eff * hide * fill);
+            // HBM reaches its sustained rate only with ~2 workgroups per CU streaming
+            const double conc = std::min(1.0, (double)blocks / (2.0 * kNumCUs));
+            // B operand streamed once per M tile (weights / cache), A once per N tile
+            // (small, mostly L2), C written once
+            const double bytes = eb * (double)p.K * p.N * p.G * std::min(tm, 2) +
+                                 ea * (double)p.M * p.K * p.G + 4.0 * (double)p.M * p.N * p.G;
+            double tt = std::max(t_mfma, bytes / (kHbm * conc));
+            if (split > 1)
+                tt += 4.0 * (split + 1) * (double)p.M * p.N * p.G / kHbm + kReduceLaunch;
+            if (tt < best_t * 0.999) {
+                best_t = tt;
+                out->bm = t.bm; out->bn = t.bn; out->split = split;
+            }
+        }
+    }
+    // A grouped fp32 NN product of short K (2c: K = 128, four slices a tile) spends a third of
+    // a tile on first loads and stores: with two rounds of tiles or more, a resident grid of
+    // two workgroups per CU walks them with its load ring running on (full tiles only, the
+    // launch checks).  2c at M = 4096: 675 -> 608-621 us.
+    const int64_t tiles = (int64_t)cdiv(p.M, out->bm) * cdiv(p.N, out->bn) * p.G;
+    if (!p.half && p.G > 1 && !p.b_nt && p.amode == kAPlain && out->split == 1 &&
+        p.K <= 8 * kBK && tiles >= 4 * kNumCUs)
+        out->tiles_per_wg = (int)((tiles + 2 * kNumCUs - 1) / (2 * kNumCUs));
+}
+
+// ---- times in us, for the comparison of the tiled engine with the large-tile one (16-bit)
+
+// Split partials written and read back, as the large-tile plan weighs its splits.
+double partials_us(const GemmProblem& p, int split) {
+    return 4.0 * (split + 1) * p.M * p.N * p.G / 3.7e6;
+}
+// The same with what a reduction launch takes; a caller that sums them itself has none.
+double split_sum_us(const GemmProblem& p, int split) {
+    if (p.sums_split) return partials_us(p, split);
+    return 1.5 + 0.25 * split + 4.0 * (split + 1) * p.M * p.N * p.G / 2.85e6;
+}
+// A tiled plan: its 64-deep slices at 0.35 us and 0.09 more per 64 x 64 of the tile on two
+// workgroups a CU (0.25 and 0.08 of it whether or not the chip is full), 4.5 us of launch, first
+// loads and stores, and at least the bytes at 3 TB/s.  Fitted to 1,109 measured products of the
+// planner's own tiled plans (M = 129..4096, N = 64..3072, K = 128..7168, 16-bit; 8% rms).
+double tiled_us(const GemmProblem& p, const GemmPlan& t) {
+    const int kslices = cdiv(p.K, 64), per = cdiv(kslices, t.split);
+    const int64_t wgs = (int64_t)cdiv(p.M, t.bm) * cdiv(p.N, t.bn) * p.G * t.split;
+    const int64_t cap = 2 * kNumCUs, left = wgs % cap;
+    const double area = t.bm * t.bn / 4096.0, slice = 0.25 + 0.08 * area, load = 0.10 + 0.10 * area;
+    double us = (double)(wgs / cap) * per * (2 * slice + load);
+    if (left) us += per * ((left > kNumCUs ? 2 : 1) * slice + load * left / cap);
+    const double bytes = (2.0 * p.K * p.N + 2.0 * p.M * p.K +
+                          (p.out_type == kOutF32 ? 4.0 : 2.0) * p.M * p.N) * p.G;
+    us = 4.5 + std::max(us, bytes / 3.0e6);
+    return t.split > 1 ? us + split_sum_us(p, t.split) : us;
+}
+
+// The 16-bit products with 16-bit A run on two more engines: up to 128 rows on the weight-streaming
+// one (wgemm.hip), past that on the large-tile one (bgemm.hip), where a product is long enough for
+// them (wgemm_short, bgemm_rule).  The line lies at one row tile
 // of the former: at M = 160 and 200 its second, nearly empty tile already costs what a full
 // one does (o_proj 98 us at M = 256 against 84-90 on the large tiles at M = 160-200), at
 // M <= 128 it is the faster one for all four weight shapes (o_proj 44-58 against 45-71 us).
@@ -807,8 +890,21 @@ bool whole_split(int kslices, int split, int* per) {
 // engine), 2a2 128 x 1 (17-22 / 31-37), o_proj 128 x 4 (44-58 / 107-117), the KV projection
 // 64 x 14 (11.4-13.7 / 14.1-16.4), 3d at M = 128 64 columns (172.4-173.1 us with the
 // attention against 174.2-175.7).
+// Short products stay on the tiled engine, whose workgroups start sooner (M = 1..128, N = 64..3072
+// unless said; it against this one): K = 128 3.6-4.6 against 3.7-5.1 us, K = 256 5.0-5.4 / 5.0-5.7,
+// K = 1024 with N = 128 6.9-8.3 / 7.3-8.7; from the line on this one: K = 512, N = 1536 6% faster,
+// K = 1536 4-25%, K = 2048 and more 10-30%.  Grouped W^T (3d, K = 512): 16 heads of 64-256 columns
+// 0.1-0.4 us slower here, 128 heads of 128 1.2-1.9 faster; 128 heads of 192, in 64-column tiles that
+// fill one and a half rounds, 0.8-1.6 slower.  Not where 2b rides on the product's epilogue.
+bool wgemm_short(const GemmProblem& p) {
+    const int64_t kn = (int64_t)p.K * p.N * p.G;
+    if (p.fuse_rope) return false;
+    if (p.G > 1) return p.b_nt && (kn < 4000000 || (p.N > 64 && p.N % 128 != 0));
+    return p.K < 1536 && (p.K <= 256 || kn < 280000);
+}
+
 bool wgemm_rule(const GemmProblem& p, GemmPlan* out) {
-    if (p.M > kStreamRows) return false;
+    if (p.M > kStreamRows || wgemm_short(p)) return false;
     const int kslices = cdiv(p.K, 64), most = max_split(p, kslices);
     double best = 1e300;
     for (int bn : {128, 64})
@@ -833,10 +929,19 @@ bool wgemm_rule(const GemmProblem& p, GemmPlan* out) {
 // lightly loaded chip, and what a full one adds as its clock drops; a workgroup (256 at a time,
 // 128 x 128: two per CU) adds ~5.6 us of launch, first loads and last stores, and ~3 us of
 // results for each further tile.  Fitted to 500 measured (shape, plan) pairs of the four weight
-// products at M = 160..4096 (9% rms; the plan it picks is within 10% of the best measured one
-// everywhere, and the best at most).  The grouped products follow it too: 3d (N = 128, K = 512)
-// takes 256 x 128 at M = 4096 (155 against 173 us on 128 x 128) and 128 x 128 at M = 256 (13.5
-// against 18), 2c (K = 128) 256 x 256 (M = 2048: 93-102 against 114 and 126).
+// products with an fp32 result at M = 160..4096 (9% rms; the plan it picks is within 10% of the
+// best measured one everywhere, and the best at most).  The grouped products follow it too: 3d
+// (N = 128, K = 512) takes 256 x 128 at M = 4096 (155 against 173 us on 128 x 128) and 128 x 128
+// at M = 256 (13.5 against 18), 2c (K = 128) 256 x 256 (M = 2048: 93-102 against 114 and 126).
+// 2a2's epilogue with 2b is not in it (128 us by it at M = 2048, 170-183 measured): it adds about
+// the same to every tile.
+//
+// The pick is then held against the tiled engine's (tiled_us), whose narrower tiles suit the small
+// products: N = 64, K = 512 at M = 129..4096 6.6-7.5 us there, 9.2-11.4 here; N = 576, K = 1536
+// 11.3 and 12.6 at M = 129, 30.5 and 18.7 at M = 4096.  Over 1,109 products (M = 129..4096,
+// N = 64..3072, K = 128..7168) the choice is 1.5% slower than the best of all plans in the mean, and
+// more than 5% slower than the tiled plan for 22 (all products here: 562).  2a2 with 2b in its
+// epilogue is not compared: on the tiled engine 2b is another launch, and 2c reads fp32.
 bool bgemm_rule(const GemmProblem& p, GemmPlan* out) {
     if (p.M <= kStreamRows) return false;
     struct Tile { int bm, bn, per_cu; double slice, load; };   // us
@@ -845,7 +950,9 @@ bool bgemm_rule(const GemmProblem& p, GemmPlan* out) {
     constexpr double kFirst = 5.6, kNext = 3.0;
     const int kslices = cdiv(p.K, 64), most = max_split(p, kslices);
     double best = 1e300;
-    for (const Tile& b : kBTiles)
+    GemmPlan pick;
+    for (const Tile& b : kBTiles) {
+        if (b.bn > 128 && p.N <= 128) continue;   // half of its columns would be empty
         for (int split = 1; split <= most; ++split) {
             int per;
             if (!whole_split(kslices, split, &per) || !bgemm_supported(p, b.bm, b.bn, split)) continue;
@@ -858,75 +965,39 @@ bool bgemm_rule(const GemmProblem& p, GemmPlan* out) {
             const double bytes = (2.0 * p.K * p.N + 2.0 * p.M * p.K +
                                   (p.out_type == kOutF32 ? 4.0 : 2.0) * p.M * p.N) * p.G;
             t = std::max(t, bytes / (5.9e6 * std::min(1.0, (double)wgs / 192)) + kFirst);
-            if (split > 1) t += 4.0 * (split + 1) * p.M * p.N * p.G / 3.7e6;
+            if (split > 1) t += partials_us(p, split);
             if (t < best * 0.999) {
                 best = t;
-                out->bm = b.bm; out->bn = b.bn; out->split = split; out->tiles_per_wg = 1;
-                out->bgemm = true;
+                pick.bm = b.bm; pick.bn = b.bn; pick.split = split;
             }
         }
-    return best < 1e300;
+    }
+    if (best == 1e300) return false;
+    if (p.fuse_rope != 64) {
+        GemmPlan tiled;
+        tiled_rule(p, &tiled);
+        if (pick.split > 1) best += split_sum_us(p, pick.split) - partials_us(p, pick.split);
+        // groups of at most half a tile's columns: 128 of 64, K = 128 at M = 512 2.3 us slower here, at
+        // M = 1024 3.9 faster
+        if (p.G > 1 && p.N <= 64) best *= 1.4;
+        if (tiled_us(p, tiled) <= best) return false;
+    }
+    *out = pick;
+    out->bgemm = true;
+    return true;
 }
 
 }  // namespace
 
 GemmPlan plan_gemm(const GemmProblem& p) {
-    // fp32 MFMA: 256 flop/clk/CU at 2.4 GHz; dense bf16 MFMA is 16x that
-    const double kCuRate = 256.0 * 2.4e9 * (p.half ? 16.0 : 1.0);
-    constexpr double kHbm = 5.0e12;             // sustained HBM B/s
-    constexpr double kReduceLaunch = 3e-6;      // s
     const int kBK = p.half ? 64 : 32;           // K per slice
-    const double eb = p.half ? 2.0 : 4.0;       // bytes per B element
-    const double ea = p.a_f32 || !p.half ? 4.0 : 2.0;
     const int kslices = cdiv(p.K, kBK);
     GemmPlan best;
-    double best_t = 1e300;
     const bool half_rules = !wgemm_off();
     if (!(half_rules && (bgemm_forced(p, &best) || wgemm_forced(p, &best))) &&
         !plan_override(p, &best) &&
-        !(half_rules && (wgemm_rule(p, &best) || bgemm_rule(p, &best))) && !tuned_plan(p, &best)) {
-        for (const auto& t : kTiles) {
-            const int tm = cdiv(p.M, t.bm), tn = cdiv(p.N, t.bn);
-            const int64_t tiles = (int64_t)tm * tn * p.G;
-            const int occ = std::max(1, std::min(2, 163840 / lds_bytes(t.bm, t.bn, p.b_nt, p.half)));
-            for (int split = 1; split <= std::max(1, kslices / 2); split *= 2) {
-                const int per = cdiv(kslices, split);
-                const int real_split = cdiv(kslices, per);
-                if (real_split != split && split > 1) continue;
-                const int64_t blocks = tiles * split;
-                // the busiest CU runs ceil(blocks / CUs) workgroups back to back or side by
-                // side; a lone workgroup per CU hides latency worse than two
-                const int64_t per_cu = (blocks + kNumCUs - 1) / kNumCUs;
-                const double hide = std::min<int64_t>(per_cu, occ) >= 2 ? 1.0 : 0.8;
-                // a workgroup's first slices and its epilogue are not overlapped with MFMA
-                // work: about four slices' worth of pipeline fill and drain
-                const double fill = per / (per + 4.0);
-                const double wg_flops = 2.0 * t.bm * t.bn * (double)per * kBK;
-                const double t_mfma = per_cu * wg_flops / (kCuRate * t.eff * hide * fill);
-                // HBM reaches its sustained rate only with ~2 workgroups per CU streaming
-                const double conc = std::min(1.0, (double)blocks / (2.0 * kNumCUs));
-                // B operand streamed once per M tile (weights / cache), A once per N tile
-                // (small, mostly L2), C written once
-                const double bytes = eb * (double)p.K * p.N * p.G * std::min(tm, 2) +
-                                     ea * (double)p.M * p.K * p.G + 4.0 * (double)p.M * p.N * p.G;
-                double tt = std::max(t_mfma, bytes / (kHbm * conc));
-                if (split > 1)
-                    tt += 4.0 * (split + 1) * (double)p.M * p.N * p.G / kHbm + kReduceLaunch;
-                if (tt < best_t * 0.999) {
-                    best_t = tt;
-                    best.bm = t.bm; best.bn = t.bn; best.split = split;
-                }
-            }
-        }
-        // A grouped fp32 NN product of short K (2c: K = 128, four slices a tile) spends a third of
-        // a tile on first loads and stores: with two rounds of tiles or more, a resident grid of
-        // two workgroups per CU walks them with its load ring running on (full tiles only, the
-        // launch checks).  2c at M = 4096: 675 -> 608-621 us.
-        const int64_t tiles = (int64_t)cdiv(p.M, best.bm) * cdiv(p.N, best.bn) * p.G;
-        if (!p.half && p.G > 1 && !p.b_nt && p.amode == kAPlain && best.split == 1 &&
-            p.K <= 8 * kBK && tiles >= 4 * kNumCUs)
-            best.tiles_per_wg = (int)((tiles + 2 * kNumCUs - 1) / (2 * kNumCUs));
-    }
+        !(half_rules && (wgemm_rule(p, &best) || bgemm_rule(p, &best))) && !tuned_plan(p, &best))
+        tiled_rule(p, &best);
     const int per = cdiv(kslices, std::max(1, std::min(best.split, kslices)));
     best.k_chunk = per * kBK;  // whole slices; the kernel's slice is the same kBK
     best.split = cdiv(kslices, per);  // no empty slices

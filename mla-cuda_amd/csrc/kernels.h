@@ -68,6 +68,10 @@ struct GemmProblem {
     const int* k_len = nullptr;
     const int* b_pages = nullptr;
     int page_size = 0, max_pages = 0;
+    // for the plan alone: the consumer sums a split's partials itself (no reduction launch); 2b can
+    // ride on the epilogue of a 16-bit engine's plan, at this many rope columns a head
+    bool sums_split = false;
+    int fuse_rope = 0;
     const QUpEpilogue* qup = nullptr;   // launch_wgemm; launch_bgemm at rope = 64, without w_uk
     // fp32 tiled plans with one K split: 2b in 2a2's epilogue (q_rope, cos_sin, H, nope,
     // rope of the struct; the nope columns still go to C)

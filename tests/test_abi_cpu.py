@@ -264,6 +264,20 @@ def test_weight_streaming_plans_size_the_workspace(lib, monkeypatch):
     assert lib.mla_gemm_workspace_bytes(BF16, 40, 200, 128) == tiled
 
 
+@pytest.mark.parametrize("M,N,K,tiled", [
+    (1, 192, 512, True), (40, 128, 512, True), (100, 64, 1024, True), (1, 576, 7168, False),
+    (129, 64, 512, True), (256, 200, 1536, True), (2048, 64, 512, True), (129, 576, 512, True),
+    (512, 128, 1536, True), (129, 1536, 7168, False), (1024, 576, 7168, False),
+    (300, 7168, 16384, False)])
+def test_short_16bit_products_stay_tiled(lib, monkeypatch, M, N, K, tiled):
+    """Products too short for the weight-streaming (M <= 128) or large tiles keep the tiled
+    engine's plan: the workspace that MLA_WGEMM=0 reports.  The long ones do not (their splits
+    differ from the tiled plan's)."""
+    got = lib.mla_gemm_workspace_bytes(BF16, M, N, K)
+    monkeypatch.setenv("MLA_WGEMM", "0")
+    assert (got == lib.mla_gemm_workspace_bytes(BF16, M, N, K)) == tiled
+
+
 @pytest.mark.parametrize("tile", ["256,256", "256,128", "128,128"])
 def test_forced_large_tiles_take_no_grouped_split(lib, monkeypatch, tile):
     """The large-tile engine splits K of ungrouped products only: MLA_BGEMM_PLAN's split is

@@ -112,6 +112,16 @@ def test_16bit_products_by_rule(ext, M, N, K):
 
 
 @pytest.mark.parametrize("dt", [BF, H16], ids=["bf16", "f16"])
+@pytest.mark.parametrize("M,N,K", [(40, 128, 512), (129, 64, 512), (333, 576, 512), (512, 128, 1536),
+                                   (3072, 128, 256), (1540, 2112, 128), (768, 576, 1536)])
+def test_16bit_products_short_of_the_large_tiles(ext, dt, M, N, K):
+    """Both sides of the line to the tiled engine, against float64 (see above)."""
+    A, W = gemm_inputs(M, N, K, dt)
+    got = ext.gemm(gpu(A), gpu(W)).cpu()
+    torch.testing.assert_close(got, (A.double() @ W.double()).float(), rtol=1e-4, atol=1e-4)
+
+
+@pytest.mark.parametrize("dt", [BF, H16], ids=["bf16", "f16"])
 @pytest.mark.parametrize("B,Sq,per_seq", [(5, 26, True), (3, 87, False), (150, 2, True),
                                            (265, 2, True)])
 def test_q_absorbed_many_rows(ext, monkeypatch, dt, B, Sq, per_seq):
