@@ -1973,8 +1973,9 @@ __global__ void __launch_bounds__(kXThreads, 1) flash32x_kernel(FlashArgs a) {
     // Queries through the ring where workgroups follow one another on a CU: 8,192 tiles of B=8
     // S=512 take 2,393 us so, 2,429 us with each score wave loading its own.  A grid that starts
     // all at once loads them directly, beside the first blocks, which the ring makes wait: B=128
-    // Sk=4989 1,240 us so, 1,243 us through the ring.
-    const bool q_ring = gridDim.x > kNumCUs;
+    // Sk=4989 1,240 us so, 1,243 us through the ring.  A list's grid is sized for its most items:
+    // what counts is the workgroups that have one.
+    const bool q_ring = (a.wl ? load_uniform(a.wl) * a.row_tiles : (int)gridDim.x) > kNumCUs;
     const uint32_t lat0 = NS * k32PeStage;
     const uint32_t pslot = kPBase + pw * 1024 + 16u * lane;   // + stage * k32XPStage
 

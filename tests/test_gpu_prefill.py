@@ -69,6 +69,24 @@ def test_paged_row_tiles_over_xcds(ext, dt, lens):
         torch.testing.assert_close(got, ref, **C.tol(dt, ref))
 
 
+@pytest.mark.parametrize("B,H", [(3, 128), (64, 128), (140, 128), (40, 43)])
+def test_paged_f32_decode_by_live_workgroups(ext, B, H):
+    """fp32 decode over a work list whose workgroups with an item start all at once (queries
+    loaded directly) or follow one another on a CU (B = 140: through the ring)."""
+    page, max_pages = 64, 3
+    g = torch.Generator().manual_seed(B)
+    qa, qr = C.layer_queries(g, B, 1, H)
+    table = torch.randperm(B * max_pages, generator=g).reshape(B, max_pages).int()
+    ck = torch.randn(B * max_pages, page, D.kv_rank, generator=g)
+    pe = torch.randn(B * max_pages, page, D.rope, generator=g)
+    wuv = torch.randn(H, D.v, D.kv_rank, generator=g) / math.sqrt(D.kv_rank)
+    sl = torch.randint(1, page * max_pages + 1, (B,), generator=g, dtype=torch.int32)
+    got = ext.mla_attention_paged(*(gpu(t) for t in (qa, qr, ck, pe, table, sl, wuv)), SCALE).cpu()
+    ref = R.mla_attention_paged(qa.double(), qr.double(), ck.double(), pe.double(), table, sl,
+                                wuv.double(), SCALE).float()
+    torch.testing.assert_close(got, ref, **C.tol(F32, ref))
+
+
 # ---- the large-tile GEMM engine
 
 def gemm_inputs(M, N, K, dt):
