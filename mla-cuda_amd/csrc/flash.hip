@@ -2545,12 +2545,14 @@ constexpr int kFStages = 4;   // LDS ring depth
 // unit(s) * rows_b + i: unit(s) = s * B + b for the uniform splits, first[b] + s for a work
 // list (whose batches of one chunk were written directly and are skipped here).
 //
-// It is bound by the partial rows' bytes (2 KB each), if enough of them are in flight:
-//   up to kMergeFew splits a wave sums a row (lane: 8 columns), all its loads going out
-//     together, and a workgroup takes rows_per_wg rows, four at a time;
+// It is bound by the partial rows' bytes (2 KB each), if enough of them are in flight.  A workgroup
+// takes rows_per_wg rows, four at a time:
+//   up to kMergeFew splits a wave sums a row (lane: 8 columns), the loads of four splits together;
 //   past that the four waves share a row: the threads take its maximum, wave w sums splits
-//     w, w + 4, ... and the four sums are added in wave order.  Small batches, which have
-//     many splits and few rows, get one row per workgroup.
+//     w, w + 4, ... and the four sums are added in wave order.
+// With rows_per_wg = 1 (up to 2,048 rows, where a row of few splits per wave would leave CUs idle)
+// the four waves share every row.  Which it is depends on the row's own splits alone, also where
+// four rows lie in two batches (rows_b not a multiple of 4).
 // Both orders are fixed, so the merge is deterministic.  The rows of a single-chunk batch cost
 // one list read per workgroup: one workgroup per row took 45 us to find the 170,496 rows of a
 // prefill chunk's four sequences already written.
@@ -2591,6 +2593,45 @@ __global__ void __launch_bounds__(256) flash_merge_kernel(const float* __restric
                     S::pack2(w1[2], w1[3])};
         }
     };
+    // a row shared by the workgroup
+    auto share_row = [&](int r, int n, int64_t unit0, int64_t step) __attribute__((always_inline)) {
+        const int i = r % rows_b;
+        auto slot_of = [&](int s) { return (unit0 + s * step) * rows_b + i; };
+        float mx = -INFINITY;
+        for (int s = tid; s < n; s += 256) mx = fmaxf(mx, m[slot_of(s)]);
+        __syncthreads();   // the row before is done with red and part
+        red[tid] = mx;
+        __syncthreads();
+        #pragma unroll
+        for (int w = 128; w > 0; w >>= 1) {
+            if (tid < w) red[tid] = fmaxf(red[tid], red[tid + w]);
+            __syncthreads();
+        }
+        mx = red[0];
+        v4f acc0 = {0.f, 0.f, 0.f, 0.f}, acc1 = acc0;
+        float ls = 0.f;
+        for (int s = wave; s < n; s += 4) {
+            const int64_t slot = slot_of(s);
+            const float ms = m[slot];
+            const float w = ms == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(ms - mx);
+            const v4f* src = reinterpret_cast<const v4f*>(o + slot * kFR) + 2 * lane;
+            acc0 += w * src[0];
+            acc1 += w * src[1];
+            ls += w * l[slot];
+        }
+        part[wave][lane][0] = acc0;
+        part[wave][lane][1] = acc1;
+        if (lane == 0) lpart[wave] = ls;
+        __syncthreads();
+        if (wave == 0) {
+            #pragma unroll
+            for (int w = 1; w < 4; ++w) {
+                acc0 += part[w][lane][0];
+                acc1 += part[w][lane][1];
+            }
+            store(r, acc0, acc1, ((lpart[0] + lpart[1]) + lpart[2]) + lpart[3]);
+        }
+    };
     const int r_end = min(rows, ((int)blockIdx.x + 1) * rows_per_wg);
     for (int r0 = blockIdx.x * rows_per_wg, next; r0 < r_end; r0 = next) {
         int64_t unit0, step;
@@ -2602,52 +2643,20 @@ __global__ void __launch_bounds__(256) flash_merge_kernel(const float* __restric
         next = r0 + 4;
         const int last = min(next, r_end) - 1;
         const bool one_batch = r0 / rows_b == last / rows_b;
-        if (rows_per_wg == 1 || (one_batch && n0 > kMergeFew)) {
-            // the workgroup, row by row
-            for (int r = r0; r <= last; ++r) {
-                const int i = r % rows_b;
-                auto slot_of = [&](int s) { return (unit0 + s * step) * rows_b + i; };
-                float mx = -INFINITY;
-                for (int s = tid; s < n0; s += 256) mx = fmaxf(mx, m[slot_of(s)]);
-                __syncthreads();   // the row before is done with red and part
-                red[tid] = mx;
-                __syncthreads();
-                #pragma unroll
-                for (int w = 128; w > 0; w >>= 1) {
-                    if (tid < w) red[tid] = fmaxf(red[tid], red[tid + w]);
-                    __syncthreads();
-                }
-                mx = red[0];
-                v4f acc0 = {0.f, 0.f, 0.f, 0.f}, acc1 = acc0;
-                float ls = 0.f;
-                for (int s = wave; s < n0; s += 4) {
-                    const int64_t slot = slot_of(s);
-                    const float ms = m[slot];
-                    const float w = ms == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(ms - mx);
-                    const v4f* src = reinterpret_cast<const v4f*>(o + slot * kFR) + 2 * lane;
-                    acc0 += w * src[0];
-                    acc1 += w * src[1];
-                    ls += w * l[slot];
-                }
-                part[wave][lane][0] = acc0;
-                part[wave][lane][1] = acc1;
-                if (lane == 0) lpart[wave] = ls;
-                __syncthreads();
-                if (wave == 0) {
-                    #pragma unroll
-                    for (int w = 1; w < 4; ++w) {
-                        acc0 += part[w][lane][0];
-                        acc1 += part[w][lane][1];
-                    }
-                    store(r, acc0, acc1, ((lpart[0] + lpart[1]) + lpart[2]) + lpart[3]);
-                }
-            }
+        if (one_batch && (rows_per_wg == 1 || n0 > kMergeFew)) {
+            for (int r = r0; r <= last; ++r) share_row(r, n0, unit0, step);
             continue;
+        }
+        if (!one_batch) {   // the rows that the workgroup shares, then the others
+            for (int r = r0; r <= last; ++r) {
+                const int n = splits_of(r, &unit0, &step);
+                if (n > kMergeFew) share_row(r, n, unit0, step);
+            }
         }
         const int r = r0 + wave;   // a wave's row
         if (r > last) continue;
         const int n = splits_of(r, &unit0, &step);
-        if (wl && n == 1) continue;
+        if ((wl && n == 1) || n > kMergeFew) continue;
         const int i = r % rows_b;
         auto slot_of = [&](int s) { return (unit0 + s * step) * rows_b + i; };
         float mx = -INFINITY;

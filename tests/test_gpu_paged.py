@@ -266,3 +266,53 @@ def test_paged_attention_full_size_ragged(ext, monkeypatch, path):
     assert torch.isfinite(out).all()
     ref = R.mla_attention_paged(qa, qr, ck, pe, table, lens, wuv, SCALE)
     torch.testing.assert_close(out, ref, **TOL)
+
+
+def merge_inputs(B, Sq, H, long_at, seed, dt):
+    """One sequence of 4,000 keys at index `long_at` among short ones (always the same
+    sequences): a work list that cuts the long one into many chunks and no other."""
+    page, long = 64, 4000
+    g = torch.Generator().manual_seed(seed)
+    pages = -(-long // page)
+    qa, qr = C.layer_queries(g, B, Sq, H)
+    ck = torch.randn(pages + B, page, D.kv_rank, generator=g)
+    pe = torch.randn(pages + B, page, D.rope, generator=g)
+    wuv = torch.randn(H, D.v, D.kv_rank, generator=g) / math.sqrt(D.kv_rank)
+    lens = torch.randint(Sq, page + 1, (B,), generator=g, dtype=torch.int32)
+    table = torch.zeros(B, pages, dtype=torch.int32)
+    table[:, 0] = torch.arange(B)
+    lens[0], table[0] = long, B + torch.randperm(pages, generator=g)
+    order = list(range(1, B))
+    order.insert(long_at, 0)
+    return tuple(t.to(dt) for t in (qa[order], qr[order], ck, pe)) + (table[order], lens[order],
+                                                                      wuv.to(dt))
+
+
+DTYPES = pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16, torch.float16],
+                                 ids=["f32", "bf16", "f16"])
+
+
+# rows = B * Sq * H: past 2,048 a workgroup merges 4 rows (H = 43: some of two sequences), from
+# 65,536 up 64, most of them of sequences that need no merge
+@DTYPES
+@pytest.mark.parametrize("B,Sq,H,long_at", [(20, 1, 128, 3), (60, 1, 43, 0), (60, 1, 43, 59),
+                                            (9, 57, 128, 4), (1541, 1, 43, 700)])
+def test_paged_merge_of_one_long_sequence(ext, dt, B, Sq, H, long_at):
+    args = merge_inputs(B, Sq, H, long_at, 7 * B + Sq, dt)
+    qa, qr, ck, pe, table, sl, wuv = args
+    got = ext.mla_attention_paged(*(gpu(t) for t in args), SCALE, Sq > 1).float().cpu()
+    pick = sorted({0, long_at, min(long_at + 1, B - 1), B - 1})
+    ref = R.mla_attention_paged(qa[pick].double(), qr[pick].double(), ck.double(), pe.double(),
+                                table[pick], sl[pick], wuv.double(), SCALE, causal=Sq > 1).float()
+    torch.testing.assert_close(got[pick], ref, **C.tol(dt, ref))
+
+
+@DTYPES
+def test_paged_merge_does_not_depend_on_the_place(ext, dt):
+    """A sequence's rows are merged in the order its own splits ask for, whether or not its
+    first or last rows share a workgroup's four with another sequence's (43 heads)."""
+    outs = []
+    for at in (0, 7, 30):
+        args = merge_inputs(60, 1, 43, at, 5, dt)
+        outs.append(ext.mla_attention_paged(*(gpu(t) for t in args), SCALE).cpu()[at])
+    assert torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[2])
