@@ -771,11 +771,11 @@ void tiled_rule(const GemmProblem& p, GemmPlan* out) {
     }
     // A grouped fp32 NN product of short K (2c: K = 128, four slices a tile) spends a third of
     // a tile on first loads and stores: with two rounds of tiles or more, a resident grid of
-    // two workgroups per CU walks them with its load ring running on (full tiles only, the
-    // launch checks).  2c at M = 4096: 675 -> 608-621 us.
+    // two workgroups per CU walks them with its load ring running on.  That kernel takes whole
+    // tiles only: 2c at M = 4096 675 -> 608-621 us, at M = 4097 a workgroup per tile as before.
     const int64_t tiles = (int64_t)cdiv(p.M, out->bm) * cdiv(p.N, out->bn) * p.G;
     if (!p.half && p.G > 1 && !p.b_nt && p.amode == kAPlain && out->split == 1 &&
-        p.K <= 8 * kBK && tiles >= 4 * kNumCUs)
+        p.K <= 8 * kBK && tiles >= 4 * kNumCUs && p.M % out->bm == 0 && p.N % out->bn == 0)
         out->tiles_per_wg = (int)((tiles + 2 * kNumCUs - 1) / (2 * kNumCUs));
 }
 
@@ -1072,7 +1072,7 @@ hipError_t launch_gemm_impl(const GemmProblem& p, const GemmPlan& plan, void* wo
         return hipErrorInvalidValue;
     const int64_t nblocks64 = (int64_t)a.tiles_m * a.tiles_n * a.G * a.split;
     if (nblocks64 <= 0 || nblocks64 > 0x7fffffff) return hipErrorInvalidValue;
-    if (plan.bgemm && bgemm_aligned(p)) {
+    if (plan.bgemm) {   // pointers that are not 16-byte aligned (the C ABI takes none) are an error there
         const hipError_t e = launch_bgemm(p, plan, a.ws, stream);
         if (e != hipSuccess || plan.split == 1 || !reduce) return e;
         return split_reduce(p, a, plan.split, stream);
