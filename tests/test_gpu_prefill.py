@@ -122,8 +122,8 @@ def test_large_tile_gemm(ext, monkeypatch, dt, M, N, K, plan):
 @pytest.mark.parametrize("M", [1, 100, 128, 129, 300, 520])
 @pytest.mark.parametrize("N,K", [(576, 7168), (1536, 640), (200, 192)])
 def test_16bit_products_by_rule(ext, M, N, K):
-    """The plans that the rules pick on both sides of the engines' line (128 rows), among
-    them columns that only the large tiles take, against float64 (see above)."""
+    """The plans that the rules pick on both sides of the engines' line (128 rows), short
+    products on the tiled engine among them (N = 200), against float64 (see above)."""
     A, W = gemm_inputs(M, N, K, BF)
     got = ext.gemm(gpu(A), gpu(W)).cpu()
     torch.testing.assert_close(got, (A.double() @ W.double()).float(), rtol=1e-4, atol=1e-4)
@@ -177,3 +177,57 @@ def test_out_projection_many_rows(ext, monkeypatch, dt, B, Sq):
     got = ext.mla_attention(*args, SCALE, Sq > 1).cpu()
     monkeypatch.setenv("MLA_WGEMM", "0")
     assert torch.equal(got, ext.mla_attention(*args, SCALE, Sq > 1).cpu())
+
+
+# ---- the large tiles' 16-bit results and groups
+
+def o_proj_inputs(rows, H, hidden, dt):
+    g = torch.Generator().manual_seed(rows + hidden)
+    attn = torch.randn(rows, 1, H, D.v, generator=g).to(dt)
+    W_o = (torch.randn(H * D.v, hidden, generator=g) / math.sqrt(H * D.v)).to(dt)
+    return attn, W_o
+
+
+@pytest.mark.parametrize("dt", [BF, H16], ids=["bf16", "f16"])
+@pytest.mark.parametrize("rows,H,hidden,plan", [
+    (129, 8, 264, "256,256,1"), (300, 8, 264, "256,128,1"), (130, 8, 136, "128,128,1"),
+    (1332, 8, 1160, "256,256,1"),    # columns a chunk past the tile, rows off it
+    (2100, 4, 392, "256,128,1"),     # more tiles than one group of eight row tiles
+    (300, 8, 264, "128,128,2"),      # fp32 partials, rounded by the reduction
+    (1332, 128, 7168, ""), (300, 128, 7168, ""), (129, 128, 7168, ""),   # the rule's own plans
+])
+def test_large_tile_16bit_results(ext, monkeypatch, dt, rows, H, hidden, plan):
+    """The output projection rounds fp32 sums once to the storage format: within half a unit in
+    the last place of the float64 result of the same 16-bit values (bf16: 8 significant bits, a
+    unit of 2^-7, half 2^-8 of the value; fp16: 11 bits, 2^-11), and the fp32 sums' own error
+    (1e-4, as for the fp32 results above)."""
+    attn, W_o = o_proj_inputs(rows, H, hidden, dt)
+    if plan:
+        monkeypatch.setenv("MLA_BGEMM_PLAN", f"{rows},{hidden},{H * D.v},1={plan}")
+    got = ext.o_proj(gpu(attn), gpu(W_o)).cpu().double()[:, 0]
+    if rows * hidden * H > 1e8:
+        pick = torch.tensor([0, 1, rows // 2, rows - 2, rows - 1])
+        got, attn = got[pick], attn[pick]
+    ref = attn.double().reshape(attn.shape[0], -1) @ W_o.double()
+    torch.testing.assert_close(got, ref, rtol=2.0 ** (-8 if dt == BF else -11), atol=1e-4)
+
+
+@pytest.mark.parametrize("dt", [BF, H16], ids=["bf16", "f16"])
+@pytest.mark.parametrize("H,B,tile", [(12, 2100, "256,256"), (12, 2100, "256,128"),
+                                      (128, 1100, "128,128"), (5, 1100, "128,128")])
+def test_grouped_large_tiles_many_rows(ext, monkeypatch, dt, H, B, tile):
+    """3d with more than eight row tiles, whose groups start at different heads (also where
+    their number is no multiple of eight): the tiled engine's bits."""
+    args = [gpu(t) for t in C.attn_inputs(B, 1, 70, H=H, seed=B + H, dt=dt)]
+    monkeypatch.setenv("MLA_BGEMM_PLAN", f"{B},{D.v},{D.kv_rank},{H}={tile},1")
+    got = ext.mla_attention(*args, SCALE).cpu()
+    monkeypatch.delenv("MLA_BGEMM_PLAN")
+    monkeypatch.setenv("MLA_WGEMM", "0")
+    assert torch.equal(got, ext.mla_attention(*args, SCALE).cpu())
+
+
+@pytest.mark.parametrize("M,N,K", [(300, 576, 7168), (129, 1536, 7168), (520, 1536, 2048)])
+def test_f16_products_by_rule(ext, M, N, K):
+    A, W = gemm_inputs(M, N, K, H16)
+    got = ext.gemm(gpu(A), gpu(W)).cpu()
+    torch.testing.assert_close(got, (A.double() @ W.double()).float(), rtol=1e-4, atol=1e-4)
