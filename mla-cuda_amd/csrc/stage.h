@@ -30,19 +30,27 @@ __device__ __forceinline__ void lds_barrier() {
 
 typedef int32_t v4i __attribute__((ext_vector_type(4)));
 
-// 16 bytes per lane from buffer offset voff + OFF (an immediate, < 4096) into LDS at
-// lds + OFF + 16*lane (gfx950 buffer_load_dwordx4 ... lds; the instruction adds the immediate to
-// both addresses).  Written as asm so that the compiler neither tracks it (it would otherwise
-// wait for every such load before any LDS read it cannot prove disjoint) nor reorders memory
-// accesses across it; the kernel waits with explicit vmcnt.
+// 16 bytes per lane from buffer offset voff into LDS at lds + 16*lane (gfx950
+// buffer_load_dwordx4 ... lds).  Written as asm so that the compiler neither tracks it
+// (it would otherwise wait for every such load before any LDS read it cannot prove
+// disjoint) nor reorders memory accesses across it; the kernel waits with explicit vmcnt.
 // An offset past the descriptor's bytes (kOob among them) returns zeros without a memory access.
 // The scalar offset is always 0: rows are kept out by the per-lane offset alone, never by how the
 // range check counts a scalar one.  Row offsets in that VGPR cost the 16-bit passes nothing
-// (prefill 2,245 -> 2,229 us); as immediates, with one address for four rows, 1.5%.
+// (prefill 2,245 -> 2,229 us); as immediates, with one address for four rows, 1.5%.  (The zero in
+// a register: as an inline constant the large-tile GEMM lost 0.4%.)
 // (m0 is a reserved register: the compiler keeps no value in it across this statement;
 // nothing else in these kernels uses m0.)
 #pragma clang diagnostic push
 #pragma clang diagnostic ignored "-Winline-asm"
+__device__ __forceinline__ void dma16(v4i rsrc, uint32_t lds, uint32_t voff) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
+                 :
+                 : "s"(lds), "v"(voff), "s"(rsrc), "s"(0u)
+                 : "memory", "m0");
+}
+// The same with an immediate offset OFF (< 4096), which the instruction adds to both addresses:
+// the bytes at voff + OFF land at lds + OFF + 16*lane.
 template <int OFF>
 __device__ __forceinline__ void dma16_imm(v4i rsrc, uint32_t lds, uint32_t voff) {
     static_assert(OFF >= 0 && OFF < 4096, "12-bit buffer offset");
@@ -52,9 +60,6 @@ __device__ __forceinline__ void dma16_imm(v4i rsrc, uint32_t lds, uint32_t voff)
                  : "memory", "m0");
 }
 #pragma clang diagnostic pop
-__device__ __forceinline__ void dma16(v4i rsrc, uint32_t lds, uint32_t voff) {
-    dma16_imm<0>(rsrc, lds, voff);
-}
 
 __device__ __forceinline__ uint32_t lds_addr(const void* p) {
     return (uint32_t)reinterpret_cast<uintptr_t>((const lds_t*)p);

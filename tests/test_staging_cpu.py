@@ -24,10 +24,14 @@ def sources():
 def test_buffer_loads_have_no_scalar_offset():
     asm, builtin = [], []
     for name, text in sources():
-        # buffer_load_dwordx4 vaddr, srsrc, soffset offen ...
-        asm += [(name, m.group(0), m.group(1).strip())
-                for m in re.finditer(r"buffer_load_\w+ %\d, %\d, ([^ ]+) offen", text)]
+        # buffer_load_dwordx4 vaddr, srsrc, soffset offen ...: 0, or an operand bound to 0u
+        for m in re.finditer(r"buffer_load_\w+ %\d, %\d, (\S+) offen[^;]*;", text):
+            soff = m.group(1)
+            if soff.startswith("%"):
+                inputs = re.findall(r'"\w"\(([^()]*)\)', m.group(0))
+                soff = inputs[int(soff[1:])]
+            asm.append((name, m.group(0), soff))
         builtin += [(name, m.group(0), m.group(1).strip())
                     for m in re.finditer(r"raw_buffer_load_\w+\(\w+, [^;]*?, ([^,;]+), \w+\)", text)]
-    assert asm and builtin
-    assert [x for x in asm + builtin if x[2] != "0"] == []
+    assert len(asm) >= 2 and builtin
+    assert [x for x in asm + builtin if x[2] not in ("0", "0u")] == []
