@@ -1,7 +1,8 @@
 // Large-tile GEMM for the 16-bit (bf16 / fp16) products of many activation rows (a prefill
 // chunk, a verify batch of hundreds of tokens): 2a1, 2a2 with 2b in its epilogue, 2c, 3d, the
 // KV projection and the output projection.  plan_gemm (gemm.hip) says where it takes over
-// from the weight-streaming engine (wgemm.hip), which is built around one 128-row tile.
+// from the weight-streaming engine (wgemm.hip), which is built around one 128-row tile, and
+// which products are too small for its tiles and stay on the tiled engine.
 //
 // What bounds it: the 16-bit matrix cores, if the operands arrive in time.  Per 16-deep K
 // step a wave of the 256 x 256 tile reads 6 fragments (6 KB) for 8 MFMAs (256 cycles), so
@@ -29,8 +30,9 @@
 //
 // Measured (bf16, tiled engine against this one): o_proj at M = 4096 1,320 -> 796 us (1,210
 // TFLOP/s, a large library product of this card 1,163); 2a2 at M = 2048 249 -> 157 us with an
-// fp32 result, 254 + 29 (2b) -> 170-179 us with 2b in its epilogue; 2a1 at M = 2048 125 -> 62 us
-// with the sum of its splits; 2c at M = 2048 214 -> 93-95 us (with a workgroup per tile 107-116),
+// fp32 result, 254 + 29 (2b) -> 170-183 us with 2b in its epilogue; 2a1 at M = 2048 144 -> 60 us
+// in 5 splits, whose sum makes 2a-n 7.8 -> 15.7 us (as a product with its reduction launch
+// 148 -> 67); 2c at M = 2048 214 -> 93-95 us (with a workgroup per tile 107-116),
 // 3d at M = 4096 195 -> 155 us (188).
 #include <algorithm>
 

@@ -701,7 +701,8 @@ __global__ void __launch_bounds__(256) out_small_kernel(const float* __restrict_
 }  // namespace
 
 namespace {
-// the split counts 2a1's plans use get the all-loads-first sum
+// 2a1's split counts up to 128 rows (16-bit 8, fp32 16) get the all-loads-first sum; the large-tile
+// plans' (5 at 2,048 rows, 7 at 1,332) are summed four loads at a time
 template <int OUT>
 hipError_t launch_rmsnorm_t(const float* in, int nsplit, int64_t split_stride, const void* gain,
                             void* out, int M, int N, float eps, hipStream_t stream,

@@ -122,7 +122,7 @@ MLA_HD int wl_bucket(int L, int chunk) {
 // quarter of it in fp32), attention with 3d, lengths uniform up to the figure: bf16 B = 61, 4,989
 // 91.5 -> 87.3 us, B = 16, 8,192 66.4 -> 59.6, B = 32, 8,192 81.2 -> 71.3; fp8 B = 32, 8,192
 // 82.6 -> 72.4; fp32 B = 128, 4,989 772 -> 744, B = 32 286 -> 226; one sequence of 4,989 keys
-// per seven of 300, B = 64: fp32 261 -> 210.  In a simulation of the dispatch over 132 length
+// per seven of 300, B = 64: fp32 245 -> 184-189.  In a simulation of the dispatch over 132 length
 // distributions (B = 5..300) the grid ends 12% sooner in 16-bit, 18% in fp32, never over 5% later.
 constexpr int kWlTries = 8;
 MLA_HD int wl_fixed_blocks(int block_keys) { return block_keys == 16 ? 4 : 11; }
